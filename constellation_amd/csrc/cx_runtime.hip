@@ -675,17 +675,20 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
     const bool dec = !prefill && n_tokens <= kTileTok && dec_path_ok(layer, top_k, route);
     PlanSizes z = plan_sizes(n_tokens, top_k, layer->n_experts, layer->has_shared);
     if (dec) z.max_items = z.max_slots;  // one item per slot (<= 16 pairs each)
-    // Calls with at least kBigPairs pairs per resident routed expert on
-    // average: the experts' weights serve hundreds of columns, so 128-pair
-    // items through the LDS-ring GEMM instead of 64-pair items that each
-    // re-stream them.  The pairs are counted on the host: exactly when the
-    // caller knows its valid routes (the wire entry point), else as every
-    // route slot, an upper bound — route tables masked to one node of
-    // several (-1 for other nodes' experts) can then take the LDS-ring path
-    // with mostly-padding tiles (correct, slower).
+    // Calls with at least kBigMinPairs pairs per resident routed expert on
+    // average take 128-pair items through the ping-pong GEMM instead of 64-pair
+    // items that each stream the expert's weights: there the matrix cores bound
+    // the work as much as HBM does.  Measured, 64-pair against 128-pair items, at
+    // 256 experts (pairs per expert: 16 / 24 / 32 / 41 / 47 / 64): 2170 against
+    // 2246, 2349 / 2404, 2592 / 2570, 2944 / 2748, 3192 / 2923 and 4040 / 3415 us
+    // a layer; at 64 experts (16 / 32 / 64): 522 / 522, 610 / 562, 917 / 741 us.
+    // The pairs are counted on the host: exactly when the caller knows its valid
+    // routes (the wire entry point), else as every route slot, an upper bound —
+    // route tables masked to one node of several (-1 for other nodes' experts)
+    // can then take it with mostly-padding tiles (correct, slower).
     const int64_t pairs = valid_routes >= 0 ? valid_routes : (int64_t)n_tokens * top_k;
-    const bool big = !dec && big_shape_ok(layer->hidden, layer->inter, in_dtype) &&
-                     pairs >= (int64_t)kBigPairs * std::max(1, layer->n_resident);
+    const bool big = !dec && pp_ok(layer->hidden, layer->inter, ctx->max_lds) &&
+                     pairs >= (int64_t)kBigMinPairs * std::max(1, layer->n_resident);
     if (big) {
         z.item_cap = kBigPairs;
         z.max_items = z.max_slots + (z.max_pairs + kBigPairs - 1) / kBigPairs;
@@ -734,11 +737,11 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
     L.max_lds = ctx->max_lds;
     {
         Span sp(ctx, "gate_up", s);
-        CX_HIP(big ? launch_gate_up_big(L, s) : launch_gate_up(L, s));
+        CX_HIP(big ? launch_gate_up_pp(L, s) : launch_gate_up(L, s));
     }
     {
         Span sp(ctx, "down", s);
-        CX_HIP(big ? launch_down_big(L, s) : launch_down(L, s));
+        CX_HIP(big ? launch_down_pp(L, s) : launch_down(L, s));
     }
     {
         Span sp(ctx, "combine", s);

@@ -251,7 +251,7 @@ CX_API int cx_route_logits(cx_ctx* ctx, double* out, int n_tokens, int n_experts
  * planner on the device, so no route ever travels to the host.
  * cx_moe_decode targets n_tokens <= 16 per launch set;
  * cx_moe_prefill targets larger chunks (grouped MFMA GEMM tiles of 16
- * tokens, up to 64 tokens per work item).  Both accept any n_tokens. */
+ * tokens, up to 128 tokens per work item).  Both accept any n_tokens. */
 CX_API int cx_moe_decode(cx_ctx* ctx, const cx_layer* layer,
                   const void* x, int in_dtype, int n_tokens,
                   const int32_t* topk_ids, const float* topk_w, int top_k,

@@ -190,6 +190,37 @@ def test_moe_many_tokens_per_expert(gpu, oracle, H, I, E, T, K, dtype, shared):
         _free(layer, experts, sh)
 
 
+@pytest.mark.parametrize("H,I,counts,dtype", [
+    (512, 512, (1, 17, 128), torch.bfloat16),          # 4 blocks: the shortest rows
+    (1024, 1024, (33, 64, 65, 16), torch.float16),
+    (1024, 512, (48, 80, 81, 129), torch.bfloat16),
+    (512, 2048, (96, 97, 112, 32), torch.bfloat16),
+    (2048, 512, (113, 127, 256, 2), torch.float16)])
+def test_item_sizes_of_the_ping_pong_gemm(gpu, oracle, H, I, counts, dtype):
+    """Experts of exactly `counts` tokens each: every column-tile count of an
+    item and its edges, one and two items per expert, against the oracle."""
+    print(f"[moe] item sizes H={H} I={I} counts={counts}", flush=True)
+    E, T = len(counts), sum(counts)
+    assert T >= 32 * E  # the rule for 128-pair items
+    layer, experts, sh, cpu, cpu_sh = _make_layer(gpu, oracle, E, H, I, seed=150 + E, shared=False)
+    try:
+        x = gpu.gen_normal(151 + T, 1, (T, H), 1.0, dtype)
+        rng = np.random.default_rng(T)
+        ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32)[:, None]
+        wts = rng.uniform(0.05, 1.0, ids.shape).astype(np.float32)
+        y, yf = gpu.moe(layer, x, torch.from_numpy(ids).cuda(), torch.from_numpy(wts).cuda(),
+                        want_f32=True, prefill=True)
+        gpu.sync()
+        ref = _oracle_moe(oracle, cpu, cpu_sh, x.float().cpu().numpy(), ids, wts)
+        yf = yf.cpu().numpy()
+        # as the other grouped paths: fp32 sums of <= 2048 products in another order
+        assert max(rel_l2(yf[t], ref[t]) for t in range(T)) < 1e-5
+        code = BF16 if dtype == torch.bfloat16 else FP16
+        assert np.array_equal(_bits(y), oracle.encode_act(yf, code, "rne"))
+    finally:
+        _free(layer, experts, sh)
+
+
 def test_many_tokens_per_resident_expert(gpu, oracle):
     """A node's share: 4 of 16 experts resident, 160 tokens x 4 routes over
     them (160 pairs per resident expert), so the LDS-ring GEMM serves the call
