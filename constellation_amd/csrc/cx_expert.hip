@@ -680,10 +680,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
     grp_gate_up_tile<NKB, F16, SINGLE, C1>(L, blockIdx.x % n_tiles, blockIdx.x / n_tiles, grp_lds);
 }
 
-template <int NKB, bool SINGLE>
+template <int NKB>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k_dn_grp(ExpertLaunch L) {
     extern __shared__ __attribute__((aligned(16))) unsigned char grp_lds[];
-    grp_down_tile<NKB, SINGLE>(L, blockIdx.x, blockIdx.y, grp_lds);
+    grp_down_tile<NKB>(L, blockIdx.x, blockIdx.y, grp_lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -953,8 +953,7 @@ bool pick_gu_grp(const ExpertLaunch& L, int items, hipStream_t s) {
 
 template <int NKB>
 void go_dn_grp(const ExpertLaunch& L, dim3 grid, hipStream_t s) {
-    if (L.table == nullptr) cx_launch((k_dn_grp<NKB, true>), grid, dim3(512), grp_dn_lds(), s, L);
-    else cx_launch((k_dn_grp<NKB, false>), grid, dim3(512), grp_dn_lds(), s, L);
+    cx_launch(k_dn_grp<NKB>, grid, dim3(512), grp_dn_lds(), s, L);
 }
 
 bool pick_dn_grp(const ExpertLaunch& L, int items, hipStream_t s) {
@@ -992,7 +991,8 @@ hipError_t launch_gate_up(const ExpertLaunch& L, hipStream_t s) {
 hipError_t launch_down(const ExpertLaunch& L, hipStream_t s) {
     const int items = L.table != nullptr ? L.max_items
                                          : (L.n_tokens + kTileTok * L.maxt - 1) / (kTileTok * L.maxt);
-    if (grp_ok(L) && pick_dn_grp(L, items, s)) return hipGetLastError();
+    // (one expert of a shape that the grouped down tiles takes the ping-pong GEMM)
+    if (L.table != nullptr && grp_ok(L) && pick_dn_grp(L, items, s)) return hipGetLastError();
     const dim3 grid(L.hidden / (kTileRows * kWaves), items);
     const bool done = L.maxt == 1 ? pick_down<1>(L, grid, s) : pick_down<4>(L, grid, s);
     if (!done) {

@@ -447,7 +447,7 @@ __device__ __forceinline__ void grp_gate_up_tile(const ExpertLaunch& L, int tile
 // ---------------------------------------------------------------------------
 // down.  NKB = inter / 128 k-blocks (<= 64).  Each wave owns 32 rows of Wd
 // (two MFMA row tiles) and reads each h fragment once for both.
-template <int NKB, int NT, bool SINGLE>
+template <int NKB, int NT>
 __device__ __forceinline__ void grp_down_item(const ExpertLaunch& L, const Unit& u, int tile,
                                               unsigned char* lds) {
     typedef Mma<false> M;
@@ -552,23 +552,22 @@ __device__ __forceinline__ void grp_down_item(const ExpertLaunch& L, const Unit&
                 const size_t p = (size_t)(u.pb + q);
                 const f32x4 v = acc[a][tt];
                 // y_part is read once, by the combine launch: streamed stores
-                if (SINGLE) store_out4(L.y, L.y_f32, p * H + row, v, L.out_dtype);
-                else __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(L.y_part + p * H + row));
+                __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(L.y_part + p * H + row));
             }
         }
     }
 }
 
-template <int NKB, bool SINGLE>
+template <int NKB>
 __device__ __forceinline__ void grp_down_tile(const ExpertLaunch& L, int tile, int item,
                                               unsigned char* lds) {
     Unit u;
-    if (!resolve_unit<SINGLE>(L, item, kGrpPairs, &u)) return;
+    if (!resolve_unit<false>(L, item, kGrpPairs, &u)) return;
     const int nt = (u.np + kTileTok - 1) / kTileTok;
-    if (nt == 1) grp_down_item<NKB, 1, SINGLE>(L, u, tile, lds);
-    else if (nt == 2) grp_down_item<NKB, 2, SINGLE>(L, u, tile, lds);
-    else if (nt == 3) grp_down_item<NKB, 3, SINGLE>(L, u, tile, lds);
-    else grp_down_item<NKB, 4, SINGLE>(L, u, tile, lds);
+    if (nt == 1) grp_down_item<NKB, 1>(L, u, tile, lds);
+    else if (nt == 2) grp_down_item<NKB, 2>(L, u, tile, lds);
+    else if (nt == 3) grp_down_item<NKB, 3>(L, u, tile, lds);
+    else grp_down_item<NKB, 4>(L, u, tile, lds);
 }
 
 }  // namespace cx

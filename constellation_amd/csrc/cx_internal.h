@@ -161,6 +161,8 @@ struct ExpertLaunch {
     int n_tokens;
     int hidden, inter;
     int maxt;                     // token tiles per item: 1 (decode) or 4 (prefill)
+    int n_cu;                     // the device's CUs (0: unknown)
+    int item_cap;                 // single mode of the ping-pong GEMM: tokens per item (set by its launchers)
     const void* x;                // [T, hidden] fp16/bf16
     int in_dtype;
     uint16_t* h_hi;               // [pairs, inter] bf16 hi part of h
@@ -181,9 +183,10 @@ struct ExpertLaunch {
 };
 
 hipError_t launch_gate_up(const ExpertLaunch& L, hipStream_t s);
-// Grouped mode with items of up to kBigPairs (128) pairs, for calls with many
-// tokens per expert (cx_pp.h): gate/up writes h, down writes y_part, as
-// launch_gate_up / launch_down do.  pp_ok: the shapes they take.
+// The ping-pong GEMM (cx_pp.h): grouped mode with items of up to kBigPairs (128)
+// pairs, for calls with many tokens per expert, and single mode; gate/up writes
+// h, down writes y_part or the output, as launch_gate_up / launch_down do.
+// pp_ok: the shapes they take.
 bool pp_ok(int hidden, int inter, int max_lds);
 hipError_t launch_gate_up_pp(const ExpertLaunch& L, hipStream_t s);
 hipError_t launch_down_pp(const ExpertLaunch& L, hipStream_t s);

@@ -1,6 +1,7 @@
 // cx_pp.h — the grouped fp8 expert MLP as two LDS-ring GEMM kernels whose two
 // waves per SIMD alternate between loading and multiplying (ping-pong), for
-// items of up to 128 pairs: prefill chunks with many tokens per expert.
+// items of up to 128 pairs: prefill chunks with many tokens per expert, and one
+// expert over more than 16 tokens.
 // Semantics: RunFusedUpGateReferenceV2 / RunDownReferenceV2
 // (expert_node_v2/backend/expert_reference_v2.cc:11-144) per expert,
 // dequantise-then-fp32, h kept to 16 significant bits (bf16 hi + lo).
@@ -388,19 +389,25 @@ __device__ __forceinline__ bool pp_item_tile(int t, int n_items, int n_rt, int* 
     return *tile < n_rt;
 }
 
+template <bool SINGLE>
 __device__ __forceinline__ bool pp_unit(const ExpertLaunch& L, int n_rt, Unit* u, int* tile) {
-    const PlanHdr hd = ld_uniform(L.plan.hdr);
-    const int n_items = L.skip_shared ? hd.n_routed_items : hd.n_items;
+    int n_items;
+    if (SINGLE) {
+        n_items = (L.n_tokens + L.item_cap - 1) / L.item_cap;
+    } else {
+        const PlanHdr hd = ld_uniform(L.plan.hdr);
+        n_items = L.skip_shared ? hd.n_routed_items : hd.n_items;
+    }
     const int t = pp_tile(n_items * n_rt);
     if (t < 0) return false;
     int item;
     if (!pp_item_tile(t, n_items, n_rt, &item, tile)) return false;
-    return resolve_unit<false>(L, item, kBigPairs, u);
+    return resolve_unit<SINGLE>(L, item, SINGLE ? L.item_cap : kBigPairs, u);
 }
 
 // ---------------------------------------------------------------------------
 // gate/up: a wave's tiles are 16 gate rows and the up rows of the same
-template <int NT, bool F16>
+template <int NT, bool F16, bool SINGLE>
 __device__ __forceinline__ void pp_gate_up_item(const ExpertLaunch& L, const Unit& u, int tile, unsigned char* lds) {
     const int H = u.e.hidden, I = u.e.inter, nkb = H / kKB;
     const int wave = wave_id(), lane = threadIdx.x & 63;
@@ -412,7 +419,8 @@ __device__ __forceinline__ void pp_gate_up_item(const ExpertLaunch& L, const Uni
     const PpW w{u.e.w_gate + ao, u.e.w_up + ao, tiled ? 2048 : kKB, tiled ? 1024 : kPpK};
     PpSrc<NT> src;
     pp_sources<NT>(src, wave, lane, [&](int t) {
-        const int tok = ldi(L.plan.pair_token + u.pb + min(t, u.np - 1));
+        const int q = u.pb + min(t, u.np - 1);
+        const int tok = SINGLE ? q : ldi(L.plan.pair_token + q);
         return static_cast<const unsigned char*>(L.x) + (size_t)tok * H * 2;
     });
     const float* scales[2] = {
@@ -425,7 +433,7 @@ __device__ __forceinline__ void pp_gate_up_item(const ExpertLaunch& L, const Uni
     for (int tt = 0; tt < NT; ++tt) {
         const int q = tt * kTileTok + c;
         if (q >= u.np) continue;
-        const float wf = L.fold_weight ? L.plan.pair_weight[u.pb + q] : 1.0f;
+        const float wf = !SINGLE && L.fold_weight ? L.plan.pair_weight[u.pb + q] : 1.0f;
         const size_t o = (size_t)(u.pb + q) * I + r0 + 4 * g;
         uint32_t hi[4], lo[4];
         float hv[4];
@@ -446,7 +454,7 @@ __device__ __forceinline__ void pp_gate_up_item(const ExpertLaunch& L, const Uni
 
 // ---------------------------------------------------------------------------
 // down: h as hi + lo planes, both multiplied with the same converted weights
-template <int NT>
+template <int NT, bool SINGLE>
 __device__ __forceinline__ void pp_down_item(const ExpertLaunch& L, const Unit& u, int tile, unsigned char* lds) {
     constexpr int MT = pp_wtiles(NT, 2), NW = 2 * NT / MT;
     const int H = u.e.hidden, I = u.e.inter, nkb = I / kKB;
@@ -484,8 +492,9 @@ __device__ __forceinline__ void pp_down_item(const ExpertLaunch& L, const Unit& 
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const f32x4 v = acc[m][tt];
+            if (SINGLE) store_out4(L.y, L.y_f32, o + m * kTileRows, v, L.out_dtype);
             // read once, by the combine launch: streamed stores
-            __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(L.y_part + o + m * kTileRows));
+            else __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(L.y_part + o + m * kTileRows));
         }
     }
 }
@@ -499,19 +508,20 @@ __device__ __forceinline__ void pp_pick(int nt, F f) {
     }
 }
 
-template <bool F16>
+template <bool F16, bool SINGLE>
 __device__ __forceinline__ void pp_gate_up(const ExpertLaunch& L, unsigned char* lds) {
     Unit u;
     int tile;
-    if (!pp_unit(L, L.inter / kPpRowsGu, &u, &tile)) return;
-    pp_pick<1>((u.np + kTileTok - 1) / kTileTok, [&](auto nt) { pp_gate_up_item<nt.value, F16>(L, u, tile, lds); });
+    if (!pp_unit<SINGLE>(L, L.inter / kPpRowsGu, &u, &tile)) return;
+    pp_pick<1>((u.np + kTileTok - 1) / kTileTok, [&](auto nt) { pp_gate_up_item<nt.value, F16, SINGLE>(L, u, tile, lds); });
 }
 
+template <bool SINGLE>
 __device__ __forceinline__ void pp_down(const ExpertLaunch& L, unsigned char* lds) {
     Unit u;
     int tile;
-    if (!pp_unit(L, L.hidden / kPpRowsDn, &u, &tile)) return;
-    pp_pick<2>((u.np + kTileTok - 1) / kTileTok, [&](auto nt) { pp_down_item<nt.value>(L, u, tile, lds); });
+    if (!pp_unit<SINGLE>(L, L.hidden / kPpRowsDn, &u, &tile)) return;
+    pp_pick<2>((u.np + kTileTok - 1) / kTileTok, [&](auto nt) { pp_down_item<nt.value, SINGLE>(L, u, tile, lds); });
 }
 
 }  // namespace cx

@@ -392,18 +392,18 @@ int lds_rows(const cx_ctx* ctx, int hidden, int max_pairs_per_item) {
 // down launch writes the output).  Shared by cx_expert_run (context scratch)
 // and cx_expert_run_static (the library's static device scratch): plan_expert
 // picks the path and states the scratch it needs, run_expert launches it.
-enum ExpertPath { kPathGeneric, kPathSmall, kPathTiles };
+enum ExpertPath { kPathGeneric, kPathSmall, kPathTiles, kPathPingPong };
 
 struct ExpertPlan {
     ExpertLaunch L;
     int path;
     size_t h_f32_bytes;   // generic path: fp32 h [T, I]
-    size_t h_plane_bytes; // tile path: each bf16 plane h_hi / h_lo [T, I]
+    size_t h_plane_bytes; // tile paths: each bf16 plane h_hi / h_lo [T, I]
     size_t gu_part_bytes; // small path: k-part gate/up sums [2][2][T][I] fp32
 };
 
 ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int n_tokens,
-                       void* y, int out_dtype, float* y_f32, int max_lds) {
+                       void* y, int out_dtype, float* y_f32, int max_lds, int n_cu) {
     ExpertPlan P{};
     const size_t TI = (size_t)n_tokens * e.inter;
     if (!fast_path_ok(e)) {
@@ -425,12 +425,16 @@ ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int
     L.out_dtype = out_dtype;
     L.np_lds = L.maxt == 1 ? lds_rows(max_lds, e.hidden, n_tokens) : 0;
     L.max_lds = max_lds;
+    L.n_cu = n_cu;
     if (expert_small_ok(L)) {
         P.path = kPathSmall;
         P.gu_part_bytes = sizeof(float) * 2 * 2 * TI;
         L.gu_kparts = 2;
     } else {
-        P.path = kPathTiles;
+        // above 16 tokens the 64-token items of the grouped kernels leave most
+        // CUs idle (16 gate/up workgroups at 17..64 tokens): 66 / 108 us at 32 /
+        // 300 tokens against 42 / 59 with the ping-pong GEMM
+        P.path = L.maxt > 1 && pp_ok(e.hidden, e.inter, max_lds) ? kPathPingPong : kPathTiles;
         P.h_plane_bytes = TI * 2;
     }
     return P;
@@ -460,11 +464,11 @@ int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* 
     L.h_lo = h_lo;
     {
         Span sp(ctx, "gate_up", s);
-        CX_HIP(launch_gate_up(L, s));
+        CX_HIP(P.path == kPathPingPong ? launch_gate_up_pp(L, s) : launch_gate_up(L, s));
     }
     {
         Span sp(ctx, "down", s);
-        CX_HIP(launch_down(L, s));
+        CX_HIP(P.path == kPathPingPong ? launch_down_pp(L, s) : launch_down(L, s));
     }
     return CX_OK;
 }
@@ -481,9 +485,10 @@ static __device__ __align__(256) unsigned char scratch[CX_STATIC_SCRATCH_BYTES];
 std::mutex g_static_mu;
 unsigned char* g_static_ptr[kMaxDevices] = {};
 int g_static_lds[kMaxDevices] = {};
+int g_static_cus[kMaxDevices] = {};
 
 // The calling thread's current device must be `device`.
-int static_scratch(int device, unsigned char** ptr, int* max_lds) {
+int static_scratch(int device, unsigned char** ptr, int* max_lds, int* n_cu) {
     std::lock_guard<std::mutex> lk(g_static_mu);
     if (g_static_ptr[device] == nullptr) {
         void* p = nullptr;
@@ -500,11 +505,18 @@ int static_scratch(int device, unsigned char** ptr, int* max_lds) {
             (void)hipGetLastError();
             lds = 65536;
         }
+        int cus = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+            (void)hipGetLastError();
+            cus = 0;
+        }
         g_static_lds[device] = lds;
+        g_static_cus[device] = cus;
         g_static_ptr[device] = static_cast<unsigned char*>(p);
     }
     *ptr = g_static_ptr[device];
     *max_lds = g_static_lds[device];
+    *n_cu = g_static_cus[device];
     return CX_OK;
 }
 
@@ -1131,7 +1143,7 @@ int cx_expert_run(cx_ctx* ctx, const cx_expert_desc* expert, const void* x, int 
     if (n_tokens <= 0 || !x || !y) return fail(CX_EINVAL, "bad n_tokens or NULL buffer");
     if ((rc = set_device(ctx->device))) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->max_lds);
+    ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->max_lds, ctx->n_cu);
     if (P.h_f32_bytes && (rc = ensure(&ctx->hscratch, P.h_f32_bytes, s))) return rc;
     if (P.h_plane_bytes && ((rc = ensure(&ctx->hhi, P.h_plane_bytes, s)) ||
                             (rc = ensure(&ctx->hlo, P.h_plane_bytes, s))))
@@ -1151,9 +1163,9 @@ int cx_expert_run_static(int device, const cx_expert_desc* expert, const void* x
     if (device < 0 || device >= kMaxDevices) return fail(CX_EINVAL, "invalid device %d", device);
     if ((rc = set_device(device))) return rc;
     unsigned char* base = nullptr;
-    int max_lds = 0;
-    if ((rc = static_scratch(device, &base, &max_lds))) return rc;
-    ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, max_lds);
+    int max_lds = 0, n_cu = 0;
+    if ((rc = static_scratch(device, &base, &max_lds, &n_cu))) return rc;
+    ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, max_lds, n_cu);
     // one region per path: fp32 h, or h_hi then h_lo (256-B aligned), or the part sums
     const size_t lo_off = (P.h_plane_bytes + 255) & ~(size_t)255;
     const size_t need = std::max({P.h_f32_bytes, lo_off + P.h_plane_bytes, P.gu_part_bytes});

@@ -243,6 +243,32 @@ def test_small_batch_expert_full_size(gpu, oracle, in_dt):
         e.free()
 
 
+@pytest.mark.parametrize("T,dt", [(17, FP16), (129, BF16), (300, FP16), (700, BF16), (1100, BF16), (2000, FP16)])
+def test_many_tokens_one_expert_full_size(gpu, oracle, T, dt):
+    """More than 16 tokens take the ping-pong GEMM, whose items have 1 (17 tokens)
+    to 8 (2000) column tiles by the token count; the last item is partial.  Each
+    token against the oracle-tested 16-token path, the first, last and a middle
+    one against the oracle."""
+    print(f"[expert] many tokens T={T}", flush=True)
+    from constellation_amd.engine import Expert
+    e = Expert.generate(0, 91, 0x740)
+    try:
+        tdt = torch.bfloat16 if dt == BF16 else torch.float16
+        x = gpu.gen_normal(92, T, (T, 7168), 1.0, tdt)
+        y, yf = gpu.expert_run(e, x, want_f32=True)
+        ref = torch.cat([gpu.expert_run(e, x[t:t + 16], want_f32=True)[1] for t in range(0, T, 16)])
+        torch.cuda.synchronize()
+        err = ((yf - ref).norm(dim=1) / ref.norm(dim=1)).max().item()
+        assert err < 1e-5, err  # the same products in another fp32 order
+        cpu = oracle.gen_expert(91, 0x740)
+        for t in (0, T // 2, T - 1):
+            _, want = oracle.expert_ref(cpu, x[t:t + 1].float().cpu().numpy())
+            assert rel_l2(yf[t:t + 1].cpu().numpy(), want) < 1e-5
+        assert np.array_equal(_bits(y), oracle.encode_act(yf.cpu().numpy(), dt, "rne"))
+    finally:
+        e.free()
+
+
 def test_small_batch_expert_back_to_back(gpu, oracle):
     """Calls queued without a sync between them, alternating tokens (1..4),
     two full-size experts and a small one (other tile counts; the k-part sums
