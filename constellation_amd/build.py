@@ -31,6 +31,7 @@ ARCH = os.environ.get("CX_OFFLOAD_ARCH", "gfx950")
 SOURCES = {
     "cx_runtime.hip": [],
     "cx_expert.hip": [],
+    "cx_few.hip": [],
     "cx_pp.hip": [],
     "cx_route.hip": [],
     "cx_gen.hip": ["-ffp-contract=off"],

@@ -216,6 +216,18 @@ hipError_t launch_plan(const int32_t* ids, const float* w, int n_tokens, int top
                        int item_cap, int max_items, PlanPtrs plan, int* err_flag,
                        hipStream_t s);
 
+// One expert over 5..64 tokens (single mode, cx_few.h): gate/up writes h in the
+// order the down launch reads it, few_scratch_bytes of it from L.h_hi on.  The
+// limits, one expert of 7168 x 2048, us a call: 1..4 tokens stay on the k-part
+// launches, whose rows keep their bits whatever the batch (2 tokens 12.4 against
+// 13.3, 4 tokens 14.7 against 13.4); 5 tokens 23.7 / 13.5; 64 tokens 31.4 against 41.1 with the
+// ping-pong GEMM, 65 tokens 45.4 / 41.3.
+constexpr int kFewMinTokens = 5, kFewMaxTokens = 64;
+bool few_ok(int hidden, int inter, int n_tokens);
+size_t few_scratch_bytes(int n_tokens, int inter);
+hipError_t launch_gate_up_few(const ExpertLaunch& L, hipStream_t s);
+hipError_t launch_down_few(const ExpertLaunch& L, hipStream_t s);
+
 // One expert at 1..4 tokens (single mode): gate/up as 2 k-part sums
 // (L.gu_part, L.gu_kparts = 2), then down with K split over the waves of each
 // workgroup, h finalised from the part sums.

@@ -392,13 +392,14 @@ int lds_rows(const cx_ctx* ctx, int hidden, int max_pairs_per_item) {
 // down launch writes the output).  Shared by cx_expert_run (context scratch)
 // and cx_expert_run_static (the library's static device scratch): plan_expert
 // picks the path and states the scratch it needs, run_expert launches it.
-enum ExpertPath { kPathGeneric, kPathSmall, kPathTiles, kPathPingPong };
+enum ExpertPath { kPathGeneric, kPathSmall, kPathTiles, kPathPingPong, kPathFew };
 
 struct ExpertPlan {
     ExpertLaunch L;
     int path;
     size_t h_f32_bytes;   // generic path: fp32 h [T, I]
     size_t h_plane_bytes; // tile paths: each bf16 plane h_hi / h_lo [T, I]
+    size_t h_frag_bytes;  // few-token path: h in fragment order
     size_t gu_part_bytes; // small path: k-part gate/up sums [2][2][T][I] fp32
 };
 
@@ -426,7 +427,10 @@ ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int
     L.np_lds = L.maxt == 1 ? lds_rows(max_lds, e.hidden, n_tokens) : 0;
     L.max_lds = max_lds;
     L.n_cu = n_cu;
-    if (expert_small_ok(L)) {
+    if (few_ok(e.hidden, e.inter, n_tokens)) {
+        P.path = kPathFew;
+        P.h_frag_bytes = few_scratch_bytes(n_tokens, e.inter);
+    } else if (expert_small_ok(L)) {
         P.path = kPathSmall;
         P.gu_part_bytes = sizeof(float) * 2 * 2 * TI;
         L.gu_kparts = 2;
@@ -441,7 +445,8 @@ ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int
 }
 
 // Launches a planned expert on `s`; the scratch pointers the path needs are
-// set (h_f32 / h_hi + h_lo / gu_part).  ctx (nullable) only collects timing.
+// set (h_f32 / h_hi + h_lo / h_hi for h in fragment order / gu_part).  ctx
+// (nullable) only collects timing.
 int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* x, int in_dtype,
                int n_tokens, void* y, int out_dtype, float* y_f32, float* h_f32, uint16_t* h_hi,
                uint16_t* h_lo, float* gu_part, hipStream_t s) {
@@ -462,6 +467,15 @@ int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* 
     }
     L.h_hi = h_hi;
     L.h_lo = h_lo;
+    if (P.path == kPathFew) {
+        {
+            Span sp(ctx, "gate_up", s);
+            CX_HIP(launch_gate_up_few(L, s));
+        }
+        Span sp(ctx, "down", s);
+        CX_HIP(launch_down_few(L, s));
+        return CX_OK;
+    }
     {
         Span sp(ctx, "gate_up", s);
         CX_HIP(P.path == kPathPingPong ? launch_gate_up_pp(L, s) : launch_gate_up(L, s));
@@ -1148,6 +1162,7 @@ int cx_expert_run(cx_ctx* ctx, const cx_expert_desc* expert, const void* x, int 
     if (P.h_plane_bytes && ((rc = ensure(&ctx->hhi, P.h_plane_bytes, s)) ||
                             (rc = ensure(&ctx->hlo, P.h_plane_bytes, s))))
         return rc;
+    if (P.h_frag_bytes && (rc = ensure(&ctx->hhi, P.h_frag_bytes, s))) return rc;
     if (P.gu_part_bytes && (rc = ensure(&ctx->gu_part, P.gu_part_bytes, s))) return rc;
     return run_expert(ctx, P, *expert, x, in_dtype, n_tokens, y, out_dtype, y_f32,
                       static_cast<float*>(ctx->hscratch.p), static_cast<uint16_t*>(ctx->hhi.p),
@@ -1166,9 +1181,10 @@ int cx_expert_run_static(int device, const cx_expert_desc* expert, const void* x
     int max_lds = 0, n_cu = 0;
     if ((rc = static_scratch(device, &base, &max_lds, &n_cu))) return rc;
     ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, max_lds, n_cu);
-    // one region per path: fp32 h, or h_hi then h_lo (256-B aligned), or the part sums
+    // one region per path: fp32 h, or h_hi then h_lo (256-B aligned), or h in
+    // fragment order, or the part sums
     const size_t lo_off = (P.h_plane_bytes + 255) & ~(size_t)255;
-    const size_t need = std::max({P.h_f32_bytes, lo_off + P.h_plane_bytes, P.gu_part_bytes});
+    const size_t need = std::max({P.h_f32_bytes, lo_off + P.h_plane_bytes, P.h_frag_bytes, P.gu_part_bytes});
     if (need > CX_STATIC_SCRATCH_BYTES)
         return fail(CX_EINVAL,
                     "cx_expert_run_static: %d tokens x inter %d need %zu scratch bytes, "

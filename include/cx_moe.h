@@ -175,7 +175,8 @@ CX_API int cx_expert_run(cx_ctx* ctx, const cx_expert_desc* expert,
  * process ends.  Same kernels and results as cx_expert_run.
  * Limit: the path's scratch must fit in CX_STATIC_SCRATCH_BYTES — 16 bytes
  * per (token, inter row) at 1..4 tokens, 4 bytes (plus up to 256 of
- * alignment) otherwise; at DeepSeek-V3's inter 2048 that is up to 32 tokens.
+ * alignment) otherwise, where 5..64 tokens count as the next multiple of 16;
+ * at DeepSeek-V3's inter 2048 that is up to 32 tokens.
  * A larger call returns CX_EINVAL.  Every call on one GPU shares that GPU's
  * array, so calls that overlap on one GPU (two streams, two threads) race;
  * serialise them.  Nothing in the array has to start at zero: each call

@@ -269,6 +269,38 @@ def test_many_tokens_one_expert_full_size(gpu, oracle, T, dt):
         e.free()
 
 
+@pytest.mark.parametrize("H,I,Ts", [(7168, 2048, (5, 15, 17, 33, 64)), (1024, 2048, (5, 16, 31, 48, 49)),
+                                    (512, 512, (5, 32, 47, 63, 64))])
+@pytest.mark.parametrize("dt,tiled", [(BF16, True), (FP16, False)])
+def test_few_tokens_one_expert(gpu, oracle, H, I, Ts, dt, tiled):
+    """5..64 tokens (interleaved gate/up rows, h in fragment order): one to four
+    column tiles and their edges, both weight layouts, against the oracle, and
+    the static-scratch entry point bit for bit where it accepts the call."""
+    import ctypes as C
+    from constellation_amd._lib import CX_STATIC_SCRATCH_BYTES, lib
+    from constellation_amd.engine import Expert
+    ex = oracle.gen_expert(95, 0x780, hidden=H, inter=I)
+    e = Expert.upload(0, ex["w_up"], ex["s_up"], ex["w_gate"], ex["s_gate"], ex["w_down"], ex["s_down"], tiled=tiled)
+    try:
+        for T in Ts:
+            print(f"[expert] few tokens H={H} I={I} T={T} tiled={tiled}", flush=True)
+            x = gpu.gen_normal(96, T, (T, H), 1.0, TDT[dt])
+            y, yf = gpu.expert_run(e, x, want_f32=True)
+            torch.cuda.synchronize()
+            _, want = oracle.expert_ref(ex, x.float().cpu().numpy())
+            got = yf.cpu().numpy()
+            assert max(rel_l2(got[t], want[t]) for t in range(T)) < 1e-5
+            assert np.array_equal(_bits(y), oracle.encode_act(got, dt, "rne"))
+            ys = torch.empty_like(y)
+            rc = lib().cx_expert_run_static(0, C.byref(e.desc), x.data_ptr(), dt, T, ys.data_ptr(), dt, None, 0)
+            torch.cuda.synchronize()
+            fits = (T + 15) // 16 * 16 * I * 4 <= CX_STATIC_SCRATCH_BYTES
+            assert fits == (rc == 0)
+            assert not fits or torch.equal(ys.view(torch.int16), y.view(torch.int16))
+    finally:
+        e.free()
+
+
 def test_small_batch_expert_back_to_back(gpu, oracle):
     """Calls queued without a sync between them, alternating tokens (1..4),
     two full-size experts and a small one (other tile counts; the k-part sums
