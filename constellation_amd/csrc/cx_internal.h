@@ -25,7 +25,7 @@ constexpr int kKB = 128;        // k-block: one scale per 128 columns
 constexpr int kTileRows = 16;   // MFMA 16x16x32: 16 weight rows per wave
 constexpr int kTileTok = 16;    // 16 token (pair) columns per MFMA tile
 constexpr int kBigPairs = 128;  // pairs per item of the ping-pong grouped GEMM (many tokens per expert)
-constexpr int kBigMinPairs = 32;  // ... which calls of this many pairs per resident expert take
+constexpr int kBigMinPairs = 20;  // ... which calls of this many pairs per resident expert take
 constexpr int kWaves = 4;       // waves per workgroup
 
 // ---------------------------------------------------------------------------

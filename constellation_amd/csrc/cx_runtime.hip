@@ -705,9 +705,10 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
     // average take 128-pair items through the ping-pong GEMM instead of 64-pair
     // items that each stream the expert's weights: there the matrix cores bound
     // the work as much as HBM does.  Measured, 64-pair against 128-pair items, at
-    // 256 experts (pairs per expert: 16 / 24 / 32 / 41 / 47 / 64): 2170 against
-    // 2246, 2349 / 2404, 2592 / 2570, 2944 / 2748, 3192 / 2923 and 4040 / 3415 us
-    // a layer; at 64 experts (16 / 32 / 64): 522 / 522, 610 / 562, 917 / 741 us.
+    // 256 experts (pairs per expert: 12.5 / 16 / 20 / 24 / 28 / 32 / 47 / 128):
+    // 2119 against 2142, 2169 / 2180, 2275 / 2265, 2370 / 2338, 2469 / 2409,
+    // 2636 / 2470, 3202 / 2907 and 6997 / 5753 us a layer; at 64 experts (32 / 64
+    // / 256): 599 / 561, 915 / 738, 2655 / 2109 us.
     // The pairs are counted on the host: exactly when the caller knows its valid
     // routes (the wire entry point), else as every route slot, an upper bound —
     // route tables masked to one node of several (-1 for other nodes' experts)

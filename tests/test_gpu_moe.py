@@ -221,6 +221,30 @@ def test_item_sizes_of_the_ping_pong_gemm(gpu, oracle, H, I, counts, dtype):
         _free(layer, experts, sh)
 
 
+@pytest.mark.parametrize("n,T", [(62, 156), (63, 159), (64, 160), (149, 373)])
+def test_ping_pong_tiles_over_the_xcds(gpu, oracle, n, T):
+    """n experts and the shared one, one 128-pair item each but for the shared
+    one's, four row tiles an item: fewer than 256 workgroups, 256 and a little
+    more, and 512 with a rest, so that every branch of the tile -> XCD mapping
+    is met; against the oracle."""
+    print(f"[moe] tiles over the XCDs n={n}", flush=True)
+    H, I, K = 1024, 512, 8
+    assert 20 * n <= T * K < 128 * n  # the rule for 128-pair items, one item an expert
+    layer, experts, sh, cpu, cpu_sh = _make_layer(gpu, oracle, n, H, I, seed=180 + n, shared=True)
+    try:
+        x = gpu.gen_normal(181, n, (T, H), 1.0, torch.bfloat16)
+        ids = ((np.arange(T * K) * 11) % n).astype(np.int32).reshape(T, K)
+        wts = np.random.default_rng(n).uniform(0.05, 1.0, ids.shape).astype(np.float32)
+        y, yf = gpu.moe(layer, x, torch.from_numpy(ids).cuda(), torch.from_numpy(wts).cuda(), want_f32=True)
+        gpu.sync()
+        ref = _oracle_moe(oracle, cpu, cpu_sh, x.float().cpu().numpy(), ids, wts)
+        yf = yf.cpu().numpy()
+        assert max(rel_l2(yf[t], ref[t]) for t in range(T)) < 1e-5  # as the test above
+        assert np.array_equal(_bits(y), oracle.encode_act(yf, BF16, "rne"))
+    finally:
+        _free(layer, experts, sh)
+
+
 def test_many_tokens_per_resident_expert(gpu, oracle):
     """A node's share: 4 of 16 experts resident, 160 tokens x 4 routes over
     them (160 pairs per resident expert), so the LDS-ring GEMM serves the call
