@@ -12,7 +12,7 @@
 //    streams W_r once for up to 16 tokens; k_route_logits_mfma on the fp64
 //    matrix cores from 32 tokens up), then k_route_select_small
 //    (T <= 16, one workgroup) or k_route_select (4 tokens per workgroup),
-//    then, for the grouped MoE, k_plan.
+//    then, for the grouped MoE, k_plan (up to 64 workgroups).
 //  * decode pipeline (T <= 16, E <= 256):
 //      stage 1  k_dec_logits        router logits
 //      stage 2  k_dec_select_sgu    selection + planner (workgroup 0) |
@@ -669,12 +669,11 @@ __device__ __forceinline__ bool dup_route(const int32_t* ids, int i, int top_k) 
 }
 
 // ---------------------------------------------------------------------------
-// General planner (one workgroup, any blockDim multiple of 64).  Counting
-// sort of the (token, k) assignments by expert id; slots in ascending expert
-// id, shared expert last with pairs [0, T); routed pairs from T; items of
-// <= item_cap pairs, routed items first.  The order of pairs inside a slot
-// only picks an MFMA column, which never changes a value, so the atomic
-// cursor keeps the results deterministic.  LDS: 2*E + blockDim ints.
+// Planner.  Counting sort of the (token, k) assignments by expert id; slots in
+// ascending expert id, shared expert last with pairs [0, T); routed pairs from T;
+// items of <= item_cap pairs, routed items first.  The order of pairs inside a
+// slot only picks an MFMA column, which never changes a value, so the atomic
+// cursors keep the results deterministic.
 __device__ __forceinline__ int wave_incl_scan(int v) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
@@ -685,327 +684,225 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
     return v;
 }
 
-// Exclusive scan over the workgroup (blockDim a multiple of 64, at most
-// 4096): a scan inside each wave, the waves' totals scanned by wave 0, three
-// barriers in all.  tmp: >= 129 ints.
-__device__ __forceinline__ int block_excl_scan(int v, int* tmp, int* total) {
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = blockDim.x >> 6;
-    const int incl = wave_incl_scan(v);
-    if (lane == 63) tmp[wv] = incl;
-    __syncthreads();
-    if (wv == 0) {
-        const int t = lane < nw ? tmp[lane] : 0;
-        const int ti = wave_incl_scan(t);
-        if (lane < nw) tmp[64 + lane] = ti - t;
-        if (lane == 63) tmp[128] = ti;
-    }
-    __syncthreads();
-    const int res = incl - v + tmp[64 + wv];
-    *total = tmp[128];
-    __syncthreads();
-    return res;
+constexpr int kPlanThreads = 1024;
+
+// Items of a slot of n pairs: item_cap pairs each and the rest, but of the
+// ping-pong GEMM's 128-pair items the first takes 64 where the last would
+// otherwise hold 1 to 48: a nearly empty item costs it more than half a
+// full one's time (us at hidden 7168, inter 2048, gate/up and down together, for
+// the last two items of 9 / 10 / 11 / 12 column tiles: 169 / 179 / 191 / 196 as
+// 8 + 1..4 and 161 / 170 / 186 / 196 as 4 + 5..8).  A layer of 256 experts with
+// and without it: 4096 tokens 5530 and 5660 us, 3000 tokens 4280 and 4350.
+__device__ __forceinline__ int plan_first_item(int n, int item_cap) {
+    const int rest = n % item_cap;
+    return item_cap == kBigPairs && n > item_cap && rest > 0 && rest <= 48 ? item_cap / 2 : item_cap;
 }
 
-__device__ __forceinline__ void plan_build(const int32_t* __restrict__ ids, const float* __restrict__ w,
-                           int n_tokens, int top_k, const cx_expert_desc* table, int n_experts,
-                           int has_shared, int item_cap, int max_items, const PlanPtrs& P,
-                           int* err_flag, int* sm /* 2E + blockDim */) {
-    __shared__ int s_err;
-    int* cnt = sm;
-    int* cur = sm + n_experts;
-    int* scan = sm + 2 * n_experts;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    if (tid == 0) s_err = 0;
-    for (int e = tid; e < n_experts; e += nt) cnt[e] = 0;
-    __syncthreads();
-    const int n_assign = n_tokens * top_k;
-    for (int i = tid; i < n_assign; i += nt) {
-        const int e = ids[i];
-        if (e < 0) continue;
-        if (e >= n_experts) { atomicOr(&s_err, kErrBadExpertId); continue; }
-        if (table[e].w_up == nullptr) { atomicOr(&s_err, kErrNotResident); continue; }
-        if (dup_route(ids, i, top_k)) { atomicOr(&s_err, kErrDuplicateRoute); continue; }
-        if (!route_weight_ok(w[i])) { atomicOr(&s_err, kErrBadWeight); continue; }
-        atomicAdd(&cnt[e], 1);
+// G workgroups without a word between them: each counts every expert's valid
+// routes before and from its own share of the tokens on, so it knows the place
+// of each pair of its share, and writes those pairs, the slots and items of
+// every G-th slot and its part of the shared expert's.  What bounds one
+// workgroup is its scattered 4-byte stores (three per route) and their LDS
+// cursors; the count that all repeat reads the routes from L2 in 16-byte loads.
+// us a plan, in one workgroup with the routes staged in LDS and
+// now, 8 routes a token: 17 / 64 / 256 / 1024 / 2048 tokens of one node of four
+// 9.0 -> 7.9, 10.9 -> 7.9, 12.3 -> 9.2, 29 -> 11.5, 52 -> 13.8.
+// LDS: first pair, cursor and first item of every expert (3 E ints).
+constexpr int kPlanShare = 1024;  // routes per workgroup
+constexpr int kPlanMaxWgs = 64;
+
+struct Scan3 {
+    int v[3];
+};
+
+// Exclusive scan of three ints per thread over the workgroup (blockDim a
+// multiple of 64, at most 1024); tmp: 3 * 33 ints.
+__device__ __forceinline__ Scan3 block_excl_scan3(Scan3 x, int* tmp, Scan3* total) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    Scan3 incl;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        incl.v[i] = wave_incl_scan(x.v[i]);
+        if (lane == 63) tmp[i * 33 + wv] = incl.v[i];
     }
     __syncthreads();
-    const bool shared = has_shared && table[n_experts].w_up != nullptr;
-    const int s0 = shared ? n_tokens : 0;  // first routed pair
-    const int chunk = (n_experts + nt - 1) / nt;
-    const int e0 = min(tid * chunk, n_experts), e1 = min(e0 + chunk, n_experts);
-    int my_pairs = 0, my_slots = 0;
-    for (int e = e0; e < e1; ++e) {
-        my_pairs += cnt[e];
-        my_slots += cnt[e] > 0;
-    }
-    int tot_pairs = 0, tot_slots = 0;
-    int pair_off = s0 + block_excl_scan(my_pairs, scan, &tot_pairs);
-    int slot_off = block_excl_scan(my_slots, scan, &tot_slots);
-    for (int e = e0; e < e1; ++e) {
-        cur[e] = pair_off;
-        if (cnt[e] > 0) {
-            P.slot_expert[slot_off] = e;
-            P.slot_pair_begin[slot_off] = pair_off;
-            P.slot_pair_count[slot_off] = cnt[e];
-            ++slot_off;
+    if (wv == 0) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const int t = lane < nw ? tmp[i * 33 + lane] : 0;
+            const int ti = wave_incl_scan(t);
+            if (lane < nw) tmp[i * 33 + 16 + lane] = ti - t;
+            if (lane == 63) tmp[i * 33 + 32] = ti;
         }
-        pair_off += cnt[e];
     }
     __syncthreads();
-    for (int i = tid; i < n_assign; i += nt) {
-        const int e = ids[i];
-        const int t = i / top_k, k = i - t * top_k;
+    Scan3 r;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        r.v[i] = incl.v[i] - x.v[i] + tmp[i * 33 + 16 + wv];
+        total->v[i] = tmp[i * 33 + 32];
+    }
+    return r;
+}
+
+// 16 bytes at a 4-byte aligned address (routes come from the caller)
+struct __attribute__((packed, aligned(4))) Route4 {
+    int32_t v[4];
+};
+
+__global__ __launch_bounds__(kPlanThreads) void k_plan(const int32_t* __restrict__ ids,
+                                                            const float* __restrict__ w, int n_tokens,
+                                                            int top_k, const cx_expert_desc* table,
+                                                            int n_experts, int has_shared,
+                                                            int item_cap, int max_items, PlanPtrs P,
+                                                            int* err_flag) {
+    extern __shared__ int plan_lds[];
+    __shared__ int tmp[3 * 33];
+    const int E = n_experts, T = n_tokens, K = top_k, tid = threadIdx.x, nt = blockDim.x;
+    const int G = gridDim.x, b = blockIdx.x;
+    int* cur = plan_lds;    // routes before this share; later the next pair of the share
+    int* first = cur + E;   // routes from this share on; later the expert's first pair
+    int* item = first + E;  // residency; later 2 x first item + (its first item is a half one)
+    const int share = (T + G - 1) / G, t0 = min(b * share, T), t1 = min(t0 + share, T);
+    for (int e = tid; e < E; e += nt) {
+        cur[e] = first[e] = 0;
+        item[e] = table[e].w_up != nullptr ? 1 : 0;
+    }
+    const bool shared = has_shared && table[E].w_up != nullptr;
+    const int s0 = shared ? T : 0;  // first routed pair
+    __syncthreads();
+    // 1) counts of valid routes
+    int err = 0;
+    auto check = [&](int e, float wt, bool dup) {
+        if (e < 0) return false;
+        const int bad = e >= E ? kErrBadExpertId : !item[e] ? kErrNotResident : dup ? kErrDuplicateRoute
+                        : !route_weight_ok(wt) ? kErrBadWeight : 0;
+        err |= bad;
+        return bad == 0;
+    };
+    if (K == 8) {
+        for (int t = tid; t < T; t += nt) {
+            Route4 r[2], x[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                r[h] = reinterpret_cast<const Route4*>(ids + (size_t)t * 8)[h];
+                x[h] = reinterpret_cast<const Route4*>(w + (size_t)t * 8)[h];
+            }
+            int* to = t < t0 ? cur : first;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int e = r[k >> 2].v[k & 3];
+                bool dup = false;
+#pragma unroll
+                for (int j = 0; j < k; ++j) dup |= r[j >> 2].v[j & 3] == e;
+                if (check(e, __int_as_float(x[k >> 2].v[k & 3]), dup)) atomicAdd(&to[e], 1);
+            }
+        }
+    } else {
+        for (int i = tid; i < T * K; i += nt) {
+            const int e = ids[i];
+            if (check(e, w[i], dup_route(ids, i, K))) atomicAdd(i < t0 * K ? &cur[e] : &first[e], 1);
+        }
+    }
+    if (b == 0 && err) atomicOr(err_flag, err);
+    __syncthreads();
+    // 2) places: experts [e0, e1) of this thread
+    const int chunk = (E + nt - 1) / nt;
+    const int e0 = min(tid * chunk, E), e1 = min(e0 + chunk, E);
+    Scan3 mine = {{0, 0, 0}}, tot;
+    for (int e = e0; e < e1; ++e) {
+        const int c = cur[e] + first[e];
+        mine.v[0] += c;
+        mine.v[1] += c > 0;
+        mine.v[2] += (c + item_cap - 1) / item_cap;
+    }
+    const Scan3 at = block_excl_scan3(mine, tmp, &tot);
+    int pair = s0 + at.v[0], slot = at.v[1], it = at.v[2];
+    auto put_item = [&](int i, int sl, const cx_expert_desc& e, int pb, int np) {
+        if (i >= max_items) return;
+        P.item_slot[i] = sl;
+        P.item_pair_begin[i] = pb;
+        P.item_pair_count[i] = np;
+        ItemRec& q = P.item_rec[i];
+        q.w_up = e.w_up;
+        q.w_gate = e.w_gate;
+        q.w_down = e.w_down;
+        q.s_up = e.s_up;
+        q.s_gate = e.s_gate;
+        q.s_down = e.s_down;
+        q.pb = pb;
+        q.np = np;
+        q.up_rb = e.up_rb;
+        q.gate_rb = e.gate_rb;
+        q.down_rb = e.down_rb;
+        q.gu_layout = e.gu_layout;
+        for (int j = np; j < 4; ++j) q.tok[j] = 0;  // the others: with their pairs
+    };
+    auto put_slot = [&](int sl, int e, int pb, int pc) {
+        P.slot_expert[sl] = e;
+        P.slot_pair_begin[sl] = pb;
+        P.slot_pair_count[sl] = pc;
+        P.slot_rec[sl] = SlotRec{table[e].w_down, table[e].s_down, table[e].down_rb, 0};
+    };
+    for (int e = e0; e < e1; ++e) {
+        const int c = cur[e] + first[e], half = plan_first_item(c, item_cap);
+        const int ni = (c + item_cap - 1) / item_cap;
+        if (c > 0 && slot % G == b) {
+            put_slot(slot, e, pair, c);
+            for (int o = 0, i = it, sz = half; o < c; o += sz, sz = item_cap, ++i)
+                put_item(i, slot, table[e], pair + o, min(sz, c - o));
+        }
+        cur[e] += pair;
+        first[e] = pair;
+        item[e] = c > 0 ? 2 * it + (half != item_cap ? 1 : 0) : -1;
+        pair += c;
+        slot += c > 0;
+        it += ni;
+    }
+    // the shared expert's items, dealt over the workgroups
+    const int n_slots = tot.v[1] + (shared ? 1 : 0);
+    const int sh_half = plan_first_item(T, item_cap), sh_items = shared ? (T + item_cap - 1) / item_cap : 0;
+    for (int i = b + tid * G; i < sh_items; i += nt * G) {
+        const int o = i == 0 ? 0 : sh_half + (i - 1) * item_cap;
+        put_item(tot.v[2] + i, tot.v[1], table[E], o, min(i == 0 ? sh_half : item_cap, T - o));
+    }
+    if (b == 0 && tid == 0) {
+        if (shared) put_slot(tot.v[1], E, 0, T);
+        const int all = tot.v[2] + sh_items;
+        if (all > max_items) atomicOr(err_flag, kErrPlanOverflow);
+        P.hdr->n_slots = n_slots;
+        P.hdr->n_items = min(all, max_items);
+        P.hdr->n_pairs = s0 + tot.v[0];
+        P.hdr->n_routed_slots = tot.v[1];
+        P.hdr->n_routed_items = min(tot.v[2], max_items);
+    }
+    __syncthreads();
+    // 3) this share's pairs; an expert without valid routes has none
+    auto put_token = [&](int first_item, bool split, int rank, int t) {
+        const int f = split ? item_cap / 2 : item_cap;
+        const int i = rank < f ? 0 : 1 + (rank - f) / item_cap;
+        const int j = rank < f ? rank : (rank - f) % item_cap;
+        if (j < 4 && first_item + i < max_items) P.item_rec[first_item + i].tok[j] = t;
+    };
+    for (int j = tid; j < (t1 - t0) * K; j += nt) {
+        const int i = t0 * K + j, e = ids[i], t = i / K;
         int pos = -1;
-        if (e >= 0 && e < n_experts && table[e].w_up != nullptr && !dup_route(ids, i, top_k) &&
-            route_weight_ok(w[i])) {
+        if (e >= 0 && e < E && item[e] >= 0 && !dup_route(ids, i, K) && route_weight_ok(w[i])) {
             pos = atomicAdd(&cur[e], 1);
             P.pair_token[pos] = t;
             P.pair_weight[pos] = w[i];
+            put_token(item[e] >> 1, item[e] & 1, pos - first[e], t);
         }
-        P.token_pairs[(size_t)t * (top_k + 1) + k] = pos;
+        P.token_pairs[(size_t)t * (K + 1) + (i - t * K)] = pos;
     }
-    for (int t = tid; t < n_tokens; t += nt) {
+    for (int t = t0 + tid; t < t1; t += nt) {
         if (shared) {
             P.pair_token[t] = t;
             P.pair_weight[t] = 1.0f;
+            put_token(tot.v[2], sh_half != item_cap, t, t);
         }
-        P.token_pairs[(size_t)t * (top_k + 1) + top_k] = shared ? t : -1;
+        P.token_pairs[(size_t)t * (K + 1) + K] = shared ? t : -1;
     }
-    if (shared && tid == 0) {
-        P.slot_expert[tot_slots] = n_experts;
-        P.slot_pair_begin[tot_slots] = 0;
-        P.slot_pair_count[tot_slots] = n_tokens;
-    }
-    __syncthreads();
-    const int n_slots = tot_slots + (shared ? 1 : 0);
-    const int schunk = (n_slots + nt - 1) / nt;
-    const int s0s = min(tid * schunk, n_slots), s1s = min(s0s + schunk, n_slots);
-    int my_items = 0;
-    for (int s = s0s; s < s1s; ++s) my_items += (P.slot_pair_count[s] + item_cap - 1) / item_cap;
-    int tot_items = 0;
-    int it = block_excl_scan(my_items, scan, &tot_items);
-    for (int s = s0s; s < s1s; ++s) {
-        const int pb = P.slot_pair_begin[s], pc = P.slot_pair_count[s];
-        for (int o = 0; o < pc; o += item_cap) {
-            if (it < max_items) {
-                P.item_slot[it] = s;
-                P.item_pair_begin[it] = pb + o;
-                P.item_pair_count[it] = min(item_cap, pc - o);
-            }
-            ++it;
-        }
-    }
-    // flat records for the expert kernels
-    __syncthreads();
-    for (int s = tid; s < n_slots; s += nt) {
-        const cx_expert_desc& e = table[P.slot_expert[s]];
-        P.slot_rec[s] = SlotRec{e.w_down, e.s_down, e.down_rb, 0};
-    }
-    for (int i = tid; i < min(tot_items, max_items); i += nt) {
-        const cx_expert_desc& e = table[P.slot_expert[P.item_slot[i]]];
-        const int pb = P.item_pair_begin[i], np = P.item_pair_count[i];
-        const int t0 = P.pair_token[pb];
-        const int t1 = np > 1 ? P.pair_token[pb + 1] : 0;
-        const int t2 = np > 2 ? P.pair_token[pb + 2] : 0;
-        const int t3 = np > 3 ? P.pair_token[pb + 3] : 0;
-        P.item_rec[i] = ItemRec{e.w_up, e.w_gate, e.w_down, e.s_up, e.s_gate, e.s_down, pb, np,
-                                e.up_rb, e.gate_rb, e.down_rb, e.gu_layout, {t0, t1, t2, t3}};
-    }
-    if (tid == 0) {
-        const int shared_items = shared ? (n_tokens + item_cap - 1) / item_cap : 0;
-        if (tot_items > max_items) s_err |= kErrPlanOverflow;
-        P.hdr->n_slots = n_slots;
-        P.hdr->n_items = min(tot_items, max_items);
-        P.hdr->n_pairs = s0 + tot_pairs;
-        P.hdr->n_routed_slots = tot_slots;
-        P.hdr->n_routed_items = min(tot_items - shared_items, max_items);
-        if (s_err) atomicOr(err_flag, s_err);
-    }
-}
-
-constexpr int kPlanThreads = 1024;
-
-// Staged planner: the same plan as plan_build with every input first copied
-// into LDS in one round of independent loads (routes, layer table), so the
-// passes that follow wait only on LDS and the block barriers.  Routes are
-// held as 16-bit expert ids (clamped to [-1, E]; a route found invalid is
-// set to -1 once every thread has checked its token's repeats), each
-// thread keeping its routes' validity in a 64-bit mask: up to 64 routes per
-// thread.  LDS layout: table[E+1] | ids16[n, even] | cnt[E] | cur[E] |
-// scan[nt] | slot arrays (expert, first pair, count) [E+1] each.
-constexpr int kPlanRoutesPerThread = 64;
-
-size_t plan_staged_lds(int n_assign, int n_experts, int threads) {
-    return sizeof(cx_expert_desc) * ((size_t)n_experts + 1) + 2 * (((size_t)n_assign + 1) & ~(size_t)1) +
-           sizeof(int) * (2 * (size_t)n_experts + threads + 3 * ((size_t)n_experts + 1));
-}
-
-__device__ __forceinline__ void plan_build_staged(const int32_t* __restrict__ ids,
-                                                  const float* __restrict__ w, int n_tokens,
-                                                  int top_k, const cx_expert_desc* table,
-                                                  int n_experts, int has_shared, int item_cap,
-                                                  int max_items, const PlanPtrs& P, int* err_flag,
-                                                  unsigned char* lds) {
-    __shared__ int s_err;
-    const int E = n_experts, n_assign = n_tokens * top_k;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    cx_expert_desc* tab = reinterpret_cast<cx_expert_desc*>(lds);
-    int16_t* sid = reinterpret_cast<int16_t*>(tab + E + 1);
-    int* cnt = reinterpret_cast<int*>(sid + ((n_assign + 1) & ~1));
-    int* cur = cnt + E;
-    int* scan = cur + E;
-    int* s_exp = scan + nt;
-    int* s_pb = s_exp + E + 1;
-    int* s_pc = s_pb + E + 1;
-    // 1) inputs -> LDS, one round of independent loads
-    {
-        constexpr int kChunks = sizeof(cx_expert_desc) / 16;
-        const u32x4* src = reinterpret_cast<const u32x4*>(table);
-        u32x4* dst = reinterpret_cast<u32x4*>(tab);
-        for (int i = tid; i < (E + 1) * kChunks; i += nt) dst[i] = ld16(src + i);
-        for (int i = tid; i < n_assign; i += nt) sid[i] = (int16_t)max(-1, min(ldi(ids + i), E));
-        for (int e = tid; e < E; e += nt) cnt[e] = 0;
-        if (tid == 0) s_err = 0;
-    }
-    __syncthreads();
-    // 2) validity (range, residency, repeats within the token) and counts;
-    // then invalid routes -> -1
-    uint64_t okm = 0;
-    for (int i = tid, r = 0; i < n_assign; i += nt, ++r) {
-        const int e = sid[i];
-        if (e >= 0) {
-            if (e >= E) atomicOr(&s_err, kErrBadExpertId);
-            else if (tab[e].w_up == nullptr) atomicOr(&s_err, kErrNotResident);
-            else {
-                bool dup = false;
-                for (int j = (i / top_k) * top_k; j < i; ++j) dup |= sid[j] == e;
-                if (dup) atomicOr(&s_err, kErrDuplicateRoute);
-                else if (!route_weight_ok(ldf(w + i))) atomicOr(&s_err, kErrBadWeight);
-                else {
-                    okm |= 1ull << r;
-                    atomicAdd(&cnt[e], 1);
-                }
-            }
-        }
-    }
-    __syncthreads();
-    for (int i = tid, r = 0; i < n_assign; i += nt, ++r)
-        if (!((okm >> r) & 1)) sid[i] = -1;
-    __syncthreads();
-    // 3) slots in ascending expert id (block scans over per-thread ranges)
-    const bool shared = has_shared && tab[E].w_up != nullptr;
-    const int s0 = shared ? n_tokens : 0;  // first routed pair
-    const int chunk = (E + nt - 1) / nt;
-    const int e0 = min(tid * chunk, E), e1 = min(e0 + chunk, E);
-    int my_pairs = 0, my_slots = 0;
-    for (int e = e0; e < e1; ++e) {
-        my_pairs += cnt[e];
-        my_slots += cnt[e] > 0;
-    }
-    int tot_pairs = 0, tot_slots = 0;
-    int pair_off = s0 + block_excl_scan(my_pairs, scan, &tot_pairs);
-    int slot_off = block_excl_scan(my_slots, scan, &tot_slots);
-    for (int e = e0; e < e1; ++e) {
-        cur[e] = pair_off;
-        if (cnt[e] > 0) {
-            s_exp[slot_off] = e;
-            s_pb[slot_off] = pair_off;
-            s_pc[slot_off] = cnt[e];
-            ++slot_off;
-        }
-        pair_off += cnt[e];
-    }
-    if (shared && tid == 0) {
-        s_exp[tot_slots] = E;
-        s_pb[tot_slots] = 0;
-        s_pc[tot_slots] = n_tokens;
-    }
-    __syncthreads();
-    // 4) pairs (order inside a slot only picks an MFMA column)
-    for (int i = tid; i < n_assign; i += nt) {
-        const int t = i / top_k, k = i - t * top_k;
-        int pos = -1;
-        if (sid[i] >= 0) {
-            pos = atomicAdd(&cur[sid[i]], 1);
-            P.pair_token[pos] = t;
-            P.pair_weight[pos] = w[i];
-        }
-        P.token_pairs[(size_t)t * (top_k + 1) + k] = pos;
-    }
-    for (int t = tid; t < n_tokens; t += nt) {
-        if (shared) {
-            P.pair_token[t] = t;
-            P.pair_weight[t] = 1.0f;
-        }
-        P.token_pairs[(size_t)t * (top_k + 1) + top_k] = shared ? t : -1;
-    }
-    const int n_slots = tot_slots + (shared ? 1 : 0);
-    for (int sl = tid; sl < n_slots; sl += nt) {
-        P.slot_expert[sl] = s_exp[sl];
-        P.slot_pair_begin[sl] = s_pb[sl];
-        P.slot_pair_count[sl] = s_pc[sl];
-        const cx_expert_desc& e = tab[s_exp[sl]];
-        P.slot_rec[sl] = SlotRec{e.w_down, e.s_down, e.down_rb, 0};
-    }
-    // 5) items of <= item_cap pairs, routed first, shared last
-    const int schunk = (n_slots + nt - 1) / nt;
-    const int s0s = min(tid * schunk, n_slots), s1s = min(s0s + schunk, n_slots);
-    int my_items = 0;
-    for (int sl = s0s; sl < s1s; ++sl) my_items += (s_pc[sl] + item_cap - 1) / item_cap;
-    int tot_items = 0;
-    // (the scan's barriers also complete this block's pair_token writes)
-    int it = block_excl_scan(my_items, scan, &tot_items);
-    for (int sl = s0s; sl < s1s; ++sl) {
-        const int pb = s_pb[sl], pc = s_pc[sl];
-        const cx_expert_desc& e = tab[s_exp[sl]];
-        for (int o = 0; o < pc; o += item_cap) {
-            if (it < max_items) {
-                const int np = min(item_cap, pc - o), q0 = pb + o;
-                P.item_slot[it] = sl;
-                P.item_pair_begin[it] = q0;
-                P.item_pair_count[it] = np;
-                const int t0 = P.pair_token[q0];
-                const int t1 = np > 1 ? P.pair_token[q0 + 1] : 0;
-                const int t2 = np > 2 ? P.pair_token[q0 + 2] : 0;
-                const int t3 = np > 3 ? P.pair_token[q0 + 3] : 0;
-                P.item_rec[it] = ItemRec{e.w_up, e.w_gate, e.w_down, e.s_up, e.s_gate, e.s_down,
-                                         q0, np, e.up_rb, e.gate_rb, e.down_rb, e.gu_layout, {t0, t1, t2, t3}};
-            }
-            ++it;
-        }
-    }
-    if (tid == 0) {
-        const int shared_items = shared ? (n_tokens + item_cap - 1) / item_cap : 0;
-        if (tot_items > max_items) s_err |= kErrPlanOverflow;
-        P.hdr->n_slots = n_slots;
-        P.hdr->n_items = min(tot_items, max_items);
-        P.hdr->n_pairs = s0 + tot_pairs;
-        P.hdr->n_routed_slots = tot_slots;
-        P.hdr->n_routed_items = min(tot_items - shared_items, max_items);
-        if (s_err) atomicOr(err_flag, s_err);
-    }
-}
-
-__global__ __launch_bounds__(kPlanThreads) void k_plan_staged(const int32_t* __restrict__ ids,
-                                                              const float* __restrict__ w,
-                                                              int n_tokens, int top_k,
-                                                              const cx_expert_desc* table,
-                                                              int n_experts, int has_shared,
-                                                              int item_cap, int max_items,
-                                                              PlanPtrs P, int* err_flag) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char plds[];
-    plan_build_staged(ids, w, n_tokens, top_k, table, n_experts, has_shared, item_cap, max_items,
-                      P, err_flag, plds);
-}
-
-__global__ __launch_bounds__(kPlanThreads) void k_plan(const int32_t* __restrict__ ids,
-                                                       const float* __restrict__ w, int n_tokens,
-                                                       int top_k, const cx_expert_desc* table,
-                                                       int n_experts, int has_shared, int item_cap,
-                                                       int max_items, PlanPtrs P, int* err_flag) {
-    extern __shared__ int sm[];
-    plan_build(ids, w, n_tokens, top_k, table, n_experts, has_shared, item_cap, max_items, P,
-               err_flag, sm);
 }
 
 // ---------------------------------------------------------------------------
@@ -1013,7 +910,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(const int32_t* __restrict
 // Input: the token x expert selection in LDS (bit e of mask[t] set when
 // token t routes to expert e, with its weight wsel[t][e] and top-k position
 // ksel[t][e]) and a copy of the layer table.  Output: the same plan layout
-// as plan_build, deterministic by construction (no atomics on the order):
+// as k_plan, deterministic by construction (no atomics on the order):
 // slots in ascending expert id, a slot's pairs in ascending token order
 // starting at T (pairs [0, T) are the shared expert's), one item per slot,
 // the shared expert's slot and item last, and each pair's y_part row
@@ -1987,38 +1884,12 @@ hipError_t launch_route(const RouteArgs& R, hipStream_t s) {
                        R.item_cap, R.max_items, *R.plan, R.err_flag, s);
 }
 
-// Dynamic LDS the current device grants one workgroup (queried once per device).
-int plan_lds_limit() {
-    static std::atomic<int> cache[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
-        (void)hipGetLastError();
-        return 65536;
-    }
-    int v = cache[dev].load(std::memory_order_relaxed);
-    if (v == 0) {
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || v <= 0) {
-            (void)hipGetLastError();
-            v = 65536;
-        }
-        cache[dev].store(v, std::memory_order_relaxed);
-    }
-    return v;
-}
-
 hipError_t launch_plan(const int32_t* ids, const float* w, int n_tokens, int top_k,
                        const cx_expert_desc* table, int n_experts, int has_shared, int item_cap,
                        int max_items, PlanPtrs plan, int* err_flag, hipStream_t s) {
-    const int threads = n_tokens * top_k <= 512 ? 256 : kPlanThreads;
-    const size_t staged = plan_staged_lds(n_tokens * top_k, n_experts, threads);
-    if (n_experts < 32768 && n_tokens * top_k <= kPlanRoutesPerThread * threads &&
-        staged <= (size_t)plan_lds_limit()) {
-        cx_launch(k_plan_staged, dim3(1), dim3(threads), staged, s, ids, w, n_tokens, top_k,
-                  table, n_experts, has_shared, item_cap, max_items, plan, err_flag);
-        return hipGetLastError();
-    }
-    const size_t lds = sizeof(int) * (2 * (size_t)n_experts + threads);
-    cx_launch(k_plan, dim3(1), dim3(threads), lds, s, ids, w, n_tokens, top_k, table,
+    const int wgs = std::max(1, std::min(kPlanMaxWgs, (n_tokens * top_k + kPlanShare - 1) / kPlanShare));
+    const size_t lds = sizeof(int) * 3 * (size_t)n_experts;
+    cx_launch(k_plan, dim3(wgs), dim3(kPlanThreads), lds, s, ids, w, n_tokens, top_k, table,
               n_experts, has_shared, item_cap, max_items, plan, err_flag);
     return hipGetLastError();
 }

@@ -245,6 +245,50 @@ def test_ping_pong_tiles_over_the_xcds(gpu, oracle, n, T):
         _free(layer, experts, sh)
 
 
+@pytest.mark.parametrize("T,K,E", [(127, 8, 16), (128, 8, 16), (129, 8, 16), (257, 8, 24), (300, 5, 16), (1025, 1, 3)])
+def test_plan_over_workgroups(gpu, oracle, T, K, E):
+    """Plans of one to three workgroups around the 1024 routes that each takes,
+    8 routes a token (16-byte loads, here from a 4-byte aligned view) and other
+    counts, absent routes, experts of 129 to 1025 tokens whose first 128-pair
+    item is halved; every token against the oracle.  Then faults in the last
+    share only: dropped, and reported by the sync."""
+    print(f"[moe] plan T={T} K={K} E={E}", flush=True)
+    from constellation_amd._lib import CxError
+    H, I = 512, 512
+    layer, experts, sh, cpu, cpu_sh = _make_layer(gpu, oracle, E, H, I, seed=190 + E, shared=True)
+    try:
+        x = gpu.gen_normal(191, T, (T, H), 1.0, torch.bfloat16)
+        rng = np.random.default_rng(T)
+        ids = np.stack([rng.choice(E, K, replace=False) for _ in range(T)]).astype(np.int32)
+        ids[:, 0] = np.where(rng.random(T) < 0.2, -1, ids[:, 0])
+        wts = rng.uniform(0.05, 1.0, ids.shape).astype(np.float32)
+
+        def run(ids):
+            flat = torch.zeros(T * K + 1, dtype=torch.int32, device="cuda")
+            flat[1:] = torch.from_numpy(ids).cuda().flatten()
+            y, yf = gpu.moe(layer, x, flat[1:].view(T, K), torch.from_numpy(wts).cuda(), want_f32=True, prefill=True)
+            return yf
+
+        def check(yf, ids):
+            ref = _oracle_moe_all_tokens(oracle, experts, sh, x.float().cpu().numpy(), ids, wts)
+            yf = yf.cpu().numpy()
+            assert max(rel_l2(yf[t], ref[t]) for t in range(T)) < 1e-5  # as the other grouped paths
+
+        yf = run(ids)
+        gpu.sync()
+        check(yf, ids)
+        bad, kept = ids.copy(), ids.copy()
+        bad[-1, -1], kept[-1, -1] = E, -1
+        if K > 1:
+            bad[-2, -1], kept[-2, -1] = bad[-2, 1], -1
+        yf = run(bad)
+        with pytest.raises(CxError):
+            gpu.sync()
+        check(yf, kept)
+    finally:
+        _free(layer, experts, sh)
+
+
 def test_many_tokens_per_resident_expert(gpu, oracle):
     """A node's share: 4 of 16 experts resident, 160 tokens x 4 routes over
     them (160 pairs per resident expert), so the LDS-ring GEMM serves the call
