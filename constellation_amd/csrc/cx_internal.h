@@ -251,6 +251,7 @@ struct RouteArgs {
     int n_tokens, hidden, n_experts, n_group, topk_group, top_k, norm;
     float scale;
     double* logits;         // scratch [T, E]
+    double* part;           // scratch [route_slices, T, E] where that is above 1
     int32_t* ids;           // [T, top_k]
     float* wout;            // [T, top_k]
     // planner (nullable plan = route only)
@@ -260,6 +261,8 @@ struct RouteArgs {
     int* err_flag;
 };
 hipError_t launch_route(const RouteArgs& r, hipStream_t s);
+// K slices of the router's logits (k_route_logits_split); 0: another kernel.
+int route_slices(int n_tokens, int hidden);
 int route_max_experts();
 
 // Decode pipeline for T <= 16 tokens, E <= 256 experts.

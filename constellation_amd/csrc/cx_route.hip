@@ -8,11 +8,10 @@
 // the exact-math decision; ties break toward the lower index.
 //
 // Launch shapes
-//  * cx_route / general path: k_route_logits (one workgroup per expert row
-//    streams W_r once for up to 16 tokens; k_route_logits_mfma on the fp64
-//    matrix cores from 32 tokens up), then k_route_select_small
-//    (T <= 16, one workgroup) or k_route_select (4 tokens per workgroup),
-//    then, for the grouped MoE, k_plan (up to 64 workgroups).
+//  * cx_route / general path: k_route_logits_split (4 to 256 tokens) or
+//    k_route_logits_mfma (more), on the fp64 matrix cores, or k_route_logits (one
+//    workgroup per expert row streams W_r once for up to 16 tokens; fewer, or
+//    other widths), then k_route_select (4 tokens per workgroup), then, for the grouped MoE, k_plan (up to 64 workgroups).
 //  * decode pipeline (T <= 16, E <= 256):
 //      stage 1  k_dec_logits        router logits
 //      stage 2  k_dec_select_sgu    selection + planner (workgroup 0) |
@@ -1063,6 +1062,8 @@ struct FusedArgs {
     double* logits;
     int32_t* ids;
     float* wout;
+    const double* part;    // slices of the logits, null = logits hold them
+    int n_part;
     int epl;               // experts per lane of the register selection, 0 = LDS fallback
     // planner
     const cx_expert_desc* table;
@@ -1124,10 +1125,10 @@ constexpr int kLgE = 16;       // experts per workgroup tile
 constexpr int kLgT = 32;       // tokens per workgroup tile (two MFMA column tiles)
 constexpr int kLgWaves = 8;    // K split
 constexpr int kLgRing = 4;     // chunks in flight per wave
-constexpr int kLgMinTokens = 64;  // below: too few tiles to fill the GPU
+constexpr int kLsMinTokens = 4, kLsMaxTokens = 256;  // tokens of k_route_logits_split
 
 bool logits_mfma_ok(int n_tokens, int hidden) {
-    return n_tokens >= kLgMinTokens && hidden % (kLgWaves * 32 * kLgRing) == 0;
+    return n_tokens > kLsMaxTokens && hidden % (kLgWaves * 32 * kLgRing) == 0;
 }
 
 // 8 elements (bf16: one dwordx4; fp32: two) widened to fp64 (exact).
@@ -1222,19 +1223,91 @@ __global__ __launch_bounds__(64 * kLgWaves) void k_route_logits_mfma(FusedArgs A
     }
 }
 
-// T <= 16, selection only: wave t selects token t (register path: all tokens
-// in parallel; LDS fallback: 4 waves loop over the tokens).
-__global__ __launch_bounds__(1024) void k_route_select_small(FusedArgs A) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
-    const int wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    double* c = reinterpret_cast<double*>(dyn) + (size_t)wave * 2 * A.n_experts;
-    double* s = c + A.n_experts;
-    uint8_t* gsel = reinterpret_cast<uint8_t*>(reinterpret_cast<double*>(dyn) + 2 * (size_t)nw * A.n_experts) + wave * 64;
-    for (int t = wave; t < A.n_tokens; t += nw) {
-        select_any(A.logits + (size_t)t * A.n_experts, A.bias, A.resident, A.n_experts, A.n_group,
-                   A.topk_group, A.top_k, A.norm, A.scale, A.ids + (size_t)t * A.top_k,
-                   A.wout + (size_t)t * A.top_k, A.epl, c, s, gsel);
+// Router logits for 4 to 256 tokens: tiles of 16 experts x 16 tokens with K
+// split over S grid slices and the 4 waves of each (one accumulator for the even
+// and one for the odd MFMA steps), so that up to 256 workgroups share the
+// products: the 16 x 32 tiles above left 224 of 256 CUs idle at 64 tokens and
+// spent 24 us of matrix time on the others, and a workgroup per expert row reads
+// every token's x once per expert.  Slice z writes its sums to part[z][t][e]; the
+// selection adds them up in the order of z.  256 experts, hidden 7168, us a router
+// call before (rows up to 63 tokens, 16 x 32 tiles from 64; the selection of up to
+// 16 tokens in one workgroup) and now: 4 / 8 / 16 / 32 / 64 / 128 / 256 tokens
+// 14.8 -> 13.4, 20.4 -> 13.7, 32.1 -> 14.0, 28.4 -> 14.3, 40.8 -> 16.5, 41.8 ->
+// 20.9, 42.1 -> 30.6; 300 tokens 42.2 against 46.9 with these tiles.
+constexpr int kLsWaves = 4;
+constexpr int kLsMaxSlices = 8;
+constexpr int kLsRing = 7;  // chunks in flight per wave
+
+template <bool XF32, bool WF32>
+__global__ __launch_bounds__(64 * kLsWaves) void k_route_logits_split(FusedArgs A, double* __restrict__ part) {
+    __shared__ double red[kLsWaves][4][64];
+    const int E = A.n_experts, T = A.n_tokens, H = A.hidden;
+    const int e0 = blockIdx.x * kLgE, t0 = blockIdx.y * kTileTok;
+    const int wave = wave_id(), lane = threadIdx.x & 63;
+    const int i = lane & 15, g = lane >> 4;
+    const int nch = H / ((int)gridDim.z * kLsWaves * 32);  // 32-k chunks of this wave
+    const size_t kb = (size_t)((int)blockIdx.z * kLsWaves + wave) * nch * 32 + 8 * g;
+    const size_t wr = (size_t)min(e0 + i, E - 1) * H + kb;
+    const size_t xr = (size_t)min(t0 + i, T - 1) * H + kb;
+    f64x4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
+    Raw8<WF32> ra[kLsRing];
+    Raw8<XF32> rb[kLsRing];
+#pragma unroll
+    for (int s = 0; s < kLsRing; ++s) {
+        if (s < nch) {
+            ra[s].load(A.w, wr + (size_t)s * 32);
+            rb[s].load(A.x, xr + (size_t)s * 32);
+        }
     }
+#pragma unroll 1
+    for (int c = 0; c < nch; c += kLsRing) {
+#pragma unroll
+        for (int s = 0; s < kLsRing; ++s) {
+            if (c + s < nch) {
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[s].get(e), rb[s].get(e), acc0, 0, 0, 0);
+                    acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(ra[s].get(e + 1), rb[s].get(e + 1), acc1, 0, 0, 0);
+                }
+                if (c + s + kLsRing < nch) {
+                    ra[s].load(A.w, wr + (size_t)(c + s + kLsRing) * 32);
+                    rb[s].load(A.x, xr + (size_t)(c + s + kLsRing) * 32);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave][r][lane] = acc0[r] + acc1[r];
+    __syncthreads();
+    // thread (r, l): expert e0 + l / 16 + 4 r, token t0 + l % 16 (the f64 result layout)
+    const int r = threadIdx.x >> 6, l = threadIdx.x & 63;
+    const int t = t0 + (l & 15), e = e0 + (l >> 4) + 4 * r;
+    double v = red[0][r][l];
+#pragma unroll
+    for (int w = 1; w < kLsWaves; ++w) v += red[w][r][l];
+    if (t < T && e < E) part[((size_t)blockIdx.z * T + t) * E + e] = v;
+}
+
+// Token t's logits from the S slices, each lane those that it then selects from
+// (epl consecutive experts, or every 64th).
+__device__ __forceinline__ void sum_logits(const FusedArgs& A, int t) {
+    if (A.part == nullptr) return;
+    const int lane = threadIdx.x & 63, E = A.n_experts;
+    const size_t slice = (size_t)A.n_tokens * E, row = (size_t)t * E;
+    const int n = A.epl ? A.epl : (E + 63) / 64;
+    for (int j = 0; j < n; ++j) {
+        const int e = A.epl ? lane * A.epl + j : lane + 64 * j;
+        if (e >= E) break;
+        double p[kLsMaxSlices];
+#pragma unroll
+        for (int z = 0; z < kLsMaxSlices; ++z) p[z] = z < A.n_part ? A.part[z * slice + row + e] : 0.0;
+        double v = p[0];
+#pragma unroll
+        for (int z = 1; z < kLsMaxSlices; ++z) v += p[z];
+        A.logits[row + e] = v;
+    }
+    // the selection reads the row through restrict pointers
+    asm volatile("" ::: "memory");
 }
 
 // one wave per token, 4 tokens per workgroup
@@ -1243,6 +1316,7 @@ __global__ __launch_bounds__(kRouteThreads) void k_route_select(FusedArgs A) {
     const int wave = threadIdx.x >> 6;
     const int t = blockIdx.x * (kRouteThreads / 64) + wave;
     if (t >= A.n_tokens) return;
+    sum_logits(A, t);
     double* c = reinterpret_cast<double*>(dyn) + (size_t)wave * 2 * A.n_experts;
     double* s = c + A.n_experts;
     uint8_t* gsel = reinterpret_cast<uint8_t*>(reinterpret_cast<double*>(dyn) + 8 * (size_t)A.n_experts) + wave * 64;
@@ -1741,6 +1815,13 @@ void go_dec_plan(const DecIdsArgs& P, const ExpertLaunch* sg, hipStream_t s) {
 
 }  // namespace
 
+int route_slices(int n_tokens, int hidden) {
+    if (n_tokens < kLsMinTokens || n_tokens > kLsMaxTokens || hidden % (kLsWaves * 32) != 0) return 0;
+    int s = n_tokens <= 32 ? 8 : n_tokens <= 64 ? 4 : n_tokens <= 128 ? 2 : 1;
+    while (hidden % (kLsWaves * 32 * s) != 0) s /= 2;
+    return s;
+}
+
 bool dec_route_ok(int n_experts, int n_group) {
     const int epl = register_epl(n_experts, n_group);
     return n_experts <= kDecMaxExperts && (epl == 1 || epl == 2 || epl == 4);
@@ -1852,7 +1933,21 @@ hipError_t launch_route(const RouteArgs& R, hipStream_t s) {
     A.epl = register_epl(R.n_experts, R.n_group);
     const size_t sel = A.epl ? 0 : select_lds(R.n_experts);
     const bool xf = R.x_dtype == CX_DTYPE_F32, wf = R.w_dtype == CX_DTYPE_F32;
-    if (logits_mfma_ok(R.n_tokens, R.hidden)) {
+    const int slices = route_slices(R.n_tokens, R.hidden);
+    if (slices > 0) {
+        const dim3 lg((R.n_experts + kLgE - 1) / kLgE, (R.n_tokens + kTileTok - 1) / kTileTok, slices);
+        const dim3 blk(64 * kLsWaves);
+        double* part = slices > 1 ? R.part : R.logits;
+        if (slices > 1) {
+            if (part == nullptr) return hipErrorInvalidValue;
+            A.part = part;
+            A.n_part = slices;
+        }
+        if (xf && wf) cx_launch((k_route_logits_split<true, true>), lg, blk, 0, s, A, part);
+        else if (xf) cx_launch((k_route_logits_split<true, false>), lg, blk, 0, s, A, part);
+        else if (wf) cx_launch((k_route_logits_split<false, true>), lg, blk, 0, s, A, part);
+        else cx_launch((k_route_logits_split<false, false>), lg, blk, 0, s, A, part);
+    } else if (logits_mfma_ok(R.n_tokens, R.hidden)) {
         // many tokens: fp64 MFMA tiles
         const dim3 lg((R.n_experts + kLgE - 1) / kLgE, (R.n_tokens + kLgT - 1) / kLgT);
         const dim3 blk(64 * kLgWaves);
@@ -1870,14 +1965,7 @@ hipError_t launch_route(const RouteArgs& R, hipStream_t s) {
     }
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    if (R.n_tokens <= kRouteTB) {
-        // register path: one wave per token, all in parallel; fallback: 4 waves
-        const int threads = A.epl ? 64 * R.n_tokens : kRouteThreads;
-        const size_t lds = A.epl ? 0 : (size_t)2 * (threads / 64) * R.n_experts * sizeof(double) + (threads / 64) * 64;
-        cx_launch(k_route_select_small, dim3(1), dim3(threads), lds, s, A);
-    } else {
-        cx_launch(k_route_select, dim3((R.n_tokens + 3) / 4), dim3(kRouteThreads), sel, s, A);
-    }
+    cx_launch(k_route_select, dim3((R.n_tokens + 3) / 4), dim3(kRouteThreads), sel, s, A);
     err = hipGetLastError();
     if (err != hipSuccess || R.plan == nullptr) return err;
     return launch_plan(R.ids, R.wout, R.n_tokens, R.top_k, R.table, R.n_experts, R.has_shared,

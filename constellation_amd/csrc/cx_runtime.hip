@@ -797,7 +797,10 @@ int fill_route(cx_ctx* ctx, const void* x, int x_dtype, const void* w_router, in
         return fail(CX_EINVAL, "invalid top_k=%d for num_experts=%d", top_k, n_experts);
     int rc = set_device(ctx->device);
     if (rc) return rc;
-    if ((rc = ensure(&ctx->logits, (size_t)n_tokens * n_experts * 8, s))) return rc;
+    // the logits, then their K slices
+    const size_t cells = (size_t)n_tokens * n_experts;
+    const int slices = route_slices(n_tokens, hidden);
+    if ((rc = ensure(&ctx->logits, cells * (slices > 1 ? 1 + slices : 1) * 8, s))) return rc;
     ctx->route_T = n_tokens;
     ctx->route_E = n_experts;
     *R = RouteArgs{};
@@ -816,6 +819,7 @@ int fill_route(cx_ctx* ctx, const void* x, int x_dtype, const void* w_router, in
     R->norm = norm;
     R->scale = scale;
     R->logits = static_cast<double*>(ctx->logits.p);
+    R->part = slices > 1 ? R->logits + cells : nullptr;
     R->ids = ids;
     R->wout = wout;
     return CX_OK;

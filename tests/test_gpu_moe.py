@@ -79,6 +79,32 @@ def test_router_many_tokens_fp32_operands(gpu, oracle, xdt, wdt):
         assert np.allclose(wts[t], ow, rtol=1e-6, atol=0), t
 
 
+@pytest.mark.parametrize("E,G,H,Ts", [(256, 8, 7168, (4, 16, 17, 32, 33, 64, 65, 128, 129, 256)), (40, 1, 384, (4, 15, 130)),
+                                      (72, 8, 1024, (5, 31, 47, 127)), (64, 8, 640, (9, 64))])
+@pytest.mark.parametrize("xdt,wdt", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
+def test_router_logits_in_slices(gpu, oracle, E, G, H, Ts, xdt, wdt):
+    """Logits of 4 to 256 tokens (16 x 16 tiles, K in 8, 4, 2 or 1 slices, expert
+    and token counts that are no multiple of 16): fp64 sums of exact products, and
+    the selection made from them."""
+    for T in Ts:
+        print(f"[route] slices T={T} E={E} H={H} {xdt}", flush=True)
+        x, w, bias = _router_inputs(gpu, 400 + T, T, E, H)
+        x, w = (x.float() * 1.37).to(xdt), (w.float() * 0.73).to(wdt)
+        ids, wts = gpu.route(x, w, bias, n_group=G, topk_group=max(1, G // 2), top_k=6)
+        got = gpu.route_logits(T, E, x.device).cpu()
+        gpu.sync()
+        xd, wd = x.double().cpu(), w.double().cpu()
+        # fp64 sums of H exact products in two orders: H 2^-53 of the sum of their magnitudes each
+        assert ((got - xd @ wd.T).abs() <= 2 * H * 2.0 ** -53 * (xd.abs() @ wd.abs().T)).all(), T
+        ids, wts = ids.cpu().numpy(), wts.cpu().numpy()
+        for t, (oi, ow, margins, _) in enumerate(_oracle_route(oracle, x, w, bias, n_group=G,
+                                                               topk_group=max(1, G // 2), top_k=6)):
+            if min(margins) <= 1e-12:
+                continue  # exact-math tie: order undefined
+            assert ids[t].tolist() == oi.tolist(), (T, t)
+            assert np.allclose(wts[t], ow, rtol=1e-6, atol=0), (T, t)
+
+
 def test_router_resident_mask(gpu, oracle):
     print("[route] resident mask", flush=True)
     E, H = 64, 512
