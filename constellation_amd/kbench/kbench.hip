@@ -26,7 +26,7 @@
 //   cx_kbench one-launch   one expert, one token: k_expert_one (gate/up, grid barrier,
 //                          down in one launch) against the two launches, and the
 //                          grid barrier's own cost
-//   cx_kbench rates        per-CU rates the LDS-ring kernels are built on, in shader
+//   cx_kbench rates        per-CU rates the GEMM kernels are built on, in shader
 //                          clocks (s_memtime): ds_read_b128 bytes per clock, bf16
 //                          MFMA and fp8 -> 16-bit convert issue intervals, and
 //                          whether independent converts overlap the MFMAs
