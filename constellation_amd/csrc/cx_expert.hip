@@ -137,10 +137,10 @@ __global__ __launch_bounds__(256) void k_gate_up_rt(ExpertLaunch L) {
                 }
                 const int kn = k + D;
                 if (kn < kb1) {
-                    wb[s][0] = ld16(pg + kn * kKB);
-                    wb[s][1] = ld16(pg + kn * kKB + 16);
-                    wb[s][2] = ld16(pu + kn * kKB);
-                    wb[s][3] = ld16(pu + kn * kKB + 16);
+                    wb[s][0] = ld16(pg + kn * kw);
+                    wb[s][1] = ld16(pg + kn * kw + 16);
+                    wb[s][2] = ld16(pu + kn * kw);
+                    wb[s][3] = ld16(pu + kn * kw + 16);
                     if (MAXT == 1) {
 #pragma unroll
                         for (int j = 0; j < 4; ++j) xb[s][j] = ld16(xp[0] + kn * kKB + 8 * j);

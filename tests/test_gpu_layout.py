@@ -36,6 +36,24 @@ def _canon(w):
     return w
 
 
+def test_tiled_rows_longer_than_the_ring(gpu):
+    """A width without kernels of its own and more 128-column blocks per wave (8)
+    than its loads run ahead (4): the refill steps by the tiled layout's block."""
+    print("[layout] tiled, hidden 4096", flush=True)
+    ex = _host_expert(np.random.default_rng(9), 4096, 512)
+    rows, tile = _upload(ex, False), _upload(ex, True)
+    try:
+        for T in (1, 7, 16):
+            x = gpu.gen_normal(10, T, (T, 4096), 1.0, torch.bfloat16)
+            _, yfa = gpu.expert_run(rows, x, want_f32=True)
+            _, yfb = gpu.expert_run(tile, x, want_f32=True)
+            torch.cuda.synchronize()
+            assert torch.equal(yfa.view(torch.int32), yfb.view(torch.int32)), T
+    finally:
+        rows.free()
+        tile.free()
+
+
 def test_tiled_upload_reads_back_and_runs_like_rows(gpu):
     print("[layout] tiled upload, one expert", flush=True)
     rng = np.random.default_rng(7)
