@@ -494,8 +494,6 @@ __global__ __launch_bounds__(512) void k_gate_up_kpart(ExpertLaunch L) {
         L, blockIdx.x, 0, gk_lds, blockIdx.y);
 }
 
-constexpr int kDownKsRows = 4;   // tokens of the split-K down launch
-constexpr int kDownKsGroups = 2;  // 16-row groups per workgroup
 
 constexpr size_t down_ks_lds(int nkbw) {
     return (size_t)4 * 2 * kDownKsRows * ((size_t)nkbw * kKB * 2 + 16) + (size_t)4 * kDownKsGroups * 64 * 16;
@@ -1006,10 +1004,8 @@ hipError_t launch_down(const ExpertLaunch& L, hipStream_t s) {
 // 2 k-parts (gate/up) and 4 k ranges (down).  The launchers also need
 // L.gu_part (2 k-parts).
 bool expert_small_ok(const ExpertLaunch& L) {
-    if (L.table != nullptr || L.maxt != 1 || L.n_tokens < 1 || L.n_tokens > kDownKsRows) return false;
-    if (L.hidden % (kDownKsGroups * kTileRows) != 0) return false;
-    const int nkg = L.hidden / kKB, nkd = L.inter / kKB;
-    return (nkg == 56 || nkg == 8 || nkg == 4) && (nkd == 16 || nkd == 4);
+    return L.table == nullptr && L.maxt == 1 && L.n_tokens >= 1 && L.n_tokens <= kDownKsRows &&
+           expert_small_shape(L.hidden, L.inter);
 }
 
 namespace {

@@ -30,7 +30,6 @@ constexpr int kFewGuRows = 8;    // outputs per gate/up workgroup
 constexpr int kFewGuWaves = 8;
 constexpr int kFewDnRows = 32;
 constexpr int kFewDnWaves = 4;
-constexpr size_t kFewHBlk = 8192;  // h bytes of a 16-token tile and 128 columns: 2 planes x 4 steps x 1 KB
 
 // Gate/up: NKB blocks per wave, KSA waves with work, NT column tiles, D blocks of
 // x in flight.  x is loaded as whole rows of a block (4 tokens x 256 B an

@@ -42,18 +42,6 @@ void go_dn(const ExpertLaunch& L, hipStream_t s) {
 
 }  // namespace
 
-int few_tiles(int n_tokens) { return (n_tokens + kTileTok - 1) / kTileTok; }
-
-size_t few_scratch_bytes(int n_tokens, int inter) {
-    return (size_t)few_tiles(n_tokens) * (inter / kKB) * kFewHBlk;
-}
-
-bool few_ok(int hidden, int inter, int n_tokens) {
-    const int nkg = hidden / kKB, nkd = inter / kKB;
-    return hidden % kKB == 0 && inter % kKB == 0 && (nkg == 56 || nkg == 8 || nkg == 4) && (nkd == 16 || nkd == 4) &&
-           n_tokens >= kFewMinTokens && n_tokens <= kFewMaxTokens;
-}
-
 hipError_t launch_gate_up_few(const ExpertLaunch& L, hipStream_t s) {
     if (L.table != nullptr || !few_ok(L.hidden, L.inter, L.n_tokens)) return hipErrorInvalidValue;
     const bool f16 = L.in_dtype == CX_DTYPE_FP16;

@@ -9,6 +9,7 @@
 #include <cstdint>
 
 #include "cx_moe.h"
+#include "cx_shapes.h"
 
 namespace cx {
 
@@ -20,10 +21,6 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// Geometry of the fast grouped kernels.
-constexpr int kKB = 128;        // k-block: one scale per 128 columns
-constexpr int kTileRows = 16;   // MFMA 16x16x32: 16 weight rows per wave
-constexpr int kTileTok = 16;    // 16 token (pair) columns per MFMA tile
 constexpr int kBigPairs = 128;  // pairs per item of the ping-pong grouped GEMM (many tokens per expert)
 constexpr int kBigMinPairs = 20;  // ... which calls of this many pairs per resident expert take
 constexpr int kWaves = 4;       // waves per workgroup
@@ -45,7 +42,7 @@ struct PlanHdr {
     int n_routed_items;  // items [0, n_routed_items) belong to routed slots
     int pad[3];
 };
-constexpr int kPlanHdrInts = 8;
+static_assert(sizeof(PlanHdr) == 4 * kPlanHdrInts, "plan header");
 
 // Gate/up weight layouts (cx_expert_desc::gu_layout).  CX_LAYOUT_TILE16
 // keeps each 16-row group's k-blocks as consecutive 2 KB tiles, and inside a
@@ -90,6 +87,7 @@ struct SlotRec {
     int down_rb;
     int pad;
 };
+static_assert(sizeof(ItemRec) == kItemRecBytes && sizeof(SlotRec) == kSlotRecBytes, "plan records");
 
 struct PlanPtrs {
     PlanHdr* hdr;
@@ -216,15 +214,7 @@ hipError_t launch_plan(const int32_t* ids, const float* w, int n_tokens, int top
                        int item_cap, int max_items, PlanPtrs plan, int* err_flag,
                        hipStream_t s);
 
-// One expert over 5..64 tokens (single mode, cx_few.h): gate/up writes h in the
-// order the down launch reads it, few_scratch_bytes of it from L.h_hi on.  The
-// limits, one expert of 7168 x 2048, us a call: 1..4 tokens stay on the k-part
-// launches, whose rows keep their bits whatever the batch (2 tokens 12.4 against
-// 13.3, 4 tokens 14.7 against 13.4); 5 tokens 23.7 / 13.5; 64 tokens 31.4 against 41.1 with the
-// ping-pong GEMM, 65 tokens 45.4 / 41.3.
-constexpr int kFewMinTokens = 5, kFewMaxTokens = 64;
-bool few_ok(int hidden, int inter, int n_tokens);
-size_t few_scratch_bytes(int n_tokens, int inter);
+// One expert over 5..64 tokens (few_ok): h in fragment order from L.h_hi on.
 hipError_t launch_gate_up_few(const ExpertLaunch& L, hipStream_t s);
 hipError_t launch_down_few(const ExpertLaunch& L, hipStream_t s);
 
@@ -251,7 +241,7 @@ struct RouteArgs {
     int n_tokens, hidden, n_experts, n_group, topk_group, top_k, norm;
     float scale;
     double* logits;         // scratch [T, E]
-    double* part;           // scratch [route_slices, T, E] where that is above 1
+    double* part;           // scratch [route_slices, T, E] (launch_route, where that is above 1)
     int32_t* ids;           // [T, top_k]
     float* wout;            // [T, top_k]
     // planner (nullable plan = route only)
@@ -261,8 +251,6 @@ struct RouteArgs {
     int* err_flag;
 };
 hipError_t launch_route(const RouteArgs& r, hipStream_t s);
-// K slices of the router's logits (k_route_logits_split); 0: another kernel.
-int route_slices(int n_tokens, int hidden);
 int route_max_experts();
 
 // Decode pipeline for T <= 16 tokens, E <= 256 experts.

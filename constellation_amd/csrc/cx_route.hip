@@ -36,7 +36,6 @@ constexpr int kRouteTB = 16;        // tokens per row workgroup
 constexpr int kMaxRouteExperts = 1024;
 constexpr int kDecMaxExperts = 256;  // decode planner: one thread per expert
 constexpr int kDecThreads = 1024;    // stage-2 workgroup: 16 selection waves
-constexpr int kDecSplitMaxTokens = 8;  // the k-part split stage 2 has 8 selection waves
 
 __device__ __forceinline__ bool better(double a, int ia, double b, int ib) {
     return a > b || (a == b && ia < ib);
@@ -1125,7 +1124,6 @@ constexpr int kLgE = 16;       // experts per workgroup tile
 constexpr int kLgT = 32;       // tokens per workgroup tile (two MFMA column tiles)
 constexpr int kLgWaves = 8;    // K split
 constexpr int kLgRing = 4;     // chunks in flight per wave
-constexpr int kLsMinTokens = 4, kLsMaxTokens = 256;  // tokens of k_route_logits_split
 
 bool logits_mfma_ok(int n_tokens, int hidden) {
     return n_tokens > kLsMaxTokens && hidden % (kLgWaves * 32 * kLgRing) == 0;
@@ -1234,8 +1232,6 @@ __global__ __launch_bounds__(64 * kLgWaves) void k_route_logits_mfma(FusedArgs A
 // 16 tokens in one workgroup) and now: 4 / 8 / 16 / 32 / 64 / 128 / 256 tokens
 // 14.8 -> 13.4, 20.4 -> 13.7, 32.1 -> 14.0, 28.4 -> 14.3, 40.8 -> 16.5, 41.8 ->
 // 20.9, 42.1 -> 30.6; 300 tokens 42.2 against 46.9 with these tiles.
-constexpr int kLsWaves = 4;
-constexpr int kLsMaxSlices = 8;
 constexpr int kLsRing = 7;  // chunks in flight per wave
 
 template <bool XF32, bool WF32>
@@ -1814,13 +1810,6 @@ void go_dec_plan(const DecIdsArgs& P, const ExpertLaunch* sg, hipStream_t s) {
 }
 
 }  // namespace
-
-int route_slices(int n_tokens, int hidden) {
-    if (n_tokens < kLsMinTokens || n_tokens > kLsMaxTokens || hidden % (kLsWaves * 32) != 0) return 0;
-    int s = n_tokens <= 32 ? 8 : n_tokens <= 64 ? 4 : n_tokens <= 128 ? 2 : 1;
-    while (hidden % (kLsWaves * 32 * s) != 0) s /= 2;
-    return s;
-}
 
 bool dec_route_ok(int n_experts, int n_group) {
     const int epl = register_epl(n_experts, n_group);

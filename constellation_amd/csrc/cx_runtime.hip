@@ -231,8 +231,8 @@ struct cx_ctx {
     int* err_flag = nullptr;           // device int: error bits of the device checks
     int max_lds = 65536;               // dynamic LDS budget per workgroup
     int n_cu = 0;                      // compute units (0: unknown)
-    DevBuf plan_buf, hhi, hlo, ypart, logits, route_ids, route_w, hscratch;
-    DevBuf gu_part;                    // shared expert's k-part gate/up sums (decode)
+    DevBuf plan_buf, hhi, hlo, ypart, logits, route_part, route_ids, route_w, hscratch;
+    DevBuf gu_part;                    // k-part gate/up sums (1..4 tokens of an expert; decode's shared expert)
     DevBuf scores;                     // one-token router scores s, c [E][2] fp64 (decode)
     int route_T = 0, route_E = 0;      // shape of the fp64 logits of the last router call
     DevBuf dx, dy;                     // cx_expert_run_host staging (device)
@@ -320,29 +320,12 @@ void drain_spans(cx_ctx* ctx) {
     }
 }
 
-struct PlanSizes {
-    int max_slots, max_pairs, max_items, item_cap, maxt;
-};
-
-PlanSizes plan_sizes(int n_tokens, int top_k, int n_experts, int has_shared) {
-    PlanSizes z;
-    z.maxt = n_tokens <= kTileTok ? 1 : 4;
-    z.item_cap = kTileTok * z.maxt;
-    z.max_slots = std::min(n_tokens * top_k, n_experts) + has_shared;
-    z.max_pairs = n_tokens * top_k + n_tokens * has_shared;
-    z.max_items = z.max_slots + (z.max_pairs + z.item_cap - 1) / z.item_cap;
-    return z;
-}
-
 // dense: a decode plan (dec_plan_core), which also fills pair_row; the
 // general planner leaves it out.
-int carve_plan(cx_ctx* ctx, const PlanSizes& z, int n_tokens, int top_k, bool dense,
-               hipStream_t s, PlanPtrs* P) {
+int carve_plan(cx_ctx* ctx, const PlanSizes& z, int n_tokens, int top_k, int n_experts, int has_shared,
+               bool dense, hipStream_t s, PlanPtrs* P) {
     const size_t recs = sizeof(ItemRec) * (size_t)z.max_items + sizeof(SlotRec) * (size_t)z.max_slots;
-    const size_t ints = kPlanHdrInts + 3 * (size_t)z.max_slots + 3 * (size_t)z.max_items +
-                        2 * (size_t)z.max_pairs + (size_t)n_tokens * (top_k + 1) +
-                        (dense ? (size_t)z.max_pairs : 0);
-    int rc = ensure(&ctx->plan_buf, recs + ints * 4 + 256, s);
+    int rc = ensure(&ctx->plan_buf, plan_buffer_bytes(n_tokens, top_k, n_experts, has_shared) + 256, s);
     if (rc) return rc;
     char* raw = static_cast<char*>(ctx->plan_buf.p);
     P->item_rec = reinterpret_cast<ItemRec*>(raw);
@@ -580,8 +563,6 @@ int moe_decode(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, 
     const bool split = route != nullptr && sg != nullptr &&
                        dec_shared_split_ok(layer->hidden, layer->inter, T);
     if (split) {
-        int rc = ensure(&ctx->gu_part, sizeof(float) * 2 * 2 * (size_t)T * layer->inter, s);
-        if (rc) return rc;
         SG.gu_part = static_cast<float*>(ctx->gu_part.p);
         SG.gu_kparts = 2;
     }
@@ -598,12 +579,7 @@ int moe_decode(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, 
                        down_comb1_ok(layer->hidden, layer->inter, top_k, ctx->max_lds) &&
                        dec_fused_sel_ok(route->n_experts, route->n_group, route->topk_group,
                                         layer->hidden, top_k, route->x_dtype);
-    double* sc = nullptr;
-    if (fused) {
-        int rc = ensure(&ctx->scores, sizeof(double) * 2 * (size_t)layer->n_experts, s);
-        if (rc) return rc;
-        sc = static_cast<double*>(ctx->scores.p);
-    }
+    double* sc = fused ? static_cast<double*>(ctx->scores.p) : nullptr;
     if (route != nullptr) {
         route->plan = &P;
         route->table = layer->table;
@@ -680,6 +656,15 @@ int moe_decode(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, 
     return CX_OK;
 }
 
+// Scratch of launch_route beside the logits.
+int route_part(cx_ctx* ctx, RouteArgs* R, hipStream_t s) {
+    const size_t cells = route_part_cells(R->n_tokens, R->hidden, R->n_experts);
+    if (cells == 0) return CX_OK;
+    const int rc = ensure(&ctx->route_part, cells * sizeof(double), s);
+    R->part = static_cast<double*>(ctx->route_part.p);
+    return rc;
+}
+
 // Routed-expert compute; when `route` is given, the router runs first on the
 // same stream.  T <= 16 takes the decode pipeline where the shapes allow it;
 // otherwise route -> plan -> grouped gate/up -> per-pair down -> combine.
@@ -722,11 +707,17 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
     }
     if (z.max_pairs == 0) return fail(CX_EINVAL, "nothing to compute");
     PlanPtrs P;
-    if ((rc = carve_plan(ctx, z, n_tokens, top_k, dec, s, &P))) return rc;
+    if ((rc = carve_plan(ctx, z, n_tokens, top_k, layer->n_experts, layer->has_shared, dec, s, &P))) return rc;
     const size_t H = layer->hidden, I = layer->inter;
     if ((rc = ensure(&ctx->hhi, (size_t)z.max_pairs * I * 2, s))) return rc;
     if ((rc = ensure(&ctx->hlo, (size_t)z.max_pairs * I * 2, s))) return rc;
     if ((rc = ensure(&ctx->ypart, (size_t)z.max_pairs * H * 4, s))) return rc;
+    if (route != nullptr && dec_path_ok(layer, top_k, route)) {  // what moe_decode needs with the router
+        const size_t t = std::min(n_tokens, kDecSplitMaxTokens);
+        if ((layer->has_shared && (rc = ensure(&ctx->gu_part, sizeof(float) * 2 * 2 * t * I, s))) ||
+            (rc = ensure(&ctx->scores, sizeof(double) * 2 * (size_t)layer->n_experts, s)))
+            return rc;
+    }
     if (dec)
         return moe_decode(ctx, layer, x, in_dtype, n_tokens, ids, w, top_k, y, out_dtype, y_f32,
                           s, route, z, P);
@@ -737,6 +728,7 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
         route->item_cap = z.item_cap;
         route->max_items = z.max_items;
         route->err_flag = ctx->err_flag;
+        if ((rc = route_part(ctx, route, s))) return rc;
         Span sp(ctx, "route", s);
         CX_HIP(launch_route(*route, s));
     } else {
@@ -797,10 +789,7 @@ int fill_route(cx_ctx* ctx, const void* x, int x_dtype, const void* w_router, in
         return fail(CX_EINVAL, "invalid top_k=%d for num_experts=%d", top_k, n_experts);
     int rc = set_device(ctx->device);
     if (rc) return rc;
-    // the logits, then their K slices
-    const size_t cells = (size_t)n_tokens * n_experts;
-    const int slices = route_slices(n_tokens, hidden);
-    if ((rc = ensure(&ctx->logits, cells * (slices > 1 ? 1 + slices : 1) * 8, s))) return rc;
+    if ((rc = ensure(&ctx->logits, (size_t)n_tokens * n_experts * 8, s))) return rc;
     ctx->route_T = n_tokens;
     ctx->route_E = n_experts;
     *R = RouteArgs{};
@@ -819,7 +808,6 @@ int fill_route(cx_ctx* ctx, const void* x, int x_dtype, const void* w_router, in
     R->norm = norm;
     R->scale = scale;
     R->logits = static_cast<double*>(ctx->logits.p);
-    R->part = slices > 1 ? R->logits + cells : nullptr;
     R->ids = ids;
     R->wout = wout;
     return CX_OK;
@@ -1099,7 +1087,7 @@ int cx_ctx_destroy(cx_ctx* c) {
     (void)hipSetDevice(c->device);
     (void)hipDeviceSynchronize();
     drain_spans(c);
-    DevBuf* bufs[] = {&c->plan_buf, &c->hhi, &c->hlo, &c->ypart, &c->logits, &c->route_ids,
+    DevBuf* bufs[] = {&c->plan_buf, &c->hhi, &c->hlo, &c->ypart, &c->logits, &c->route_part, &c->route_ids,
                       &c->route_w, &c->hscratch, &c->gu_part, &c->scores, &c->dx, &c->dy};
     for (DevBuf* b : bufs)
         if (b->p) (void)hipFree(b->p);
@@ -1164,11 +1152,12 @@ int cx_expert_run(cx_ctx* ctx, const cx_expert_desc* expert, const void* x, int 
     hipStream_t s = static_cast<hipStream_t>(stream);
     ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->max_lds, ctx->n_cu);
     if (P.h_f32_bytes && (rc = ensure(&ctx->hscratch, P.h_f32_bytes, s))) return rc;
-    if (P.h_plane_bytes && ((rc = ensure(&ctx->hhi, P.h_plane_bytes, s)) ||
-                            (rc = ensure(&ctx->hlo, P.h_plane_bytes, s))))
-        return rc;
-    if (P.h_frag_bytes && (rc = ensure(&ctx->hhi, P.h_frag_bytes, s))) return rc;
-    if (P.gu_part_bytes && (rc = ensure(&ctx->gu_part, P.gu_part_bytes, s))) return rc;
+    if (P.path != kPathGeneric) {
+        const ExpertScratch z = expert_scratch(n_tokens, expert->hidden, expert->inter);
+        if ((z.h_hi && (rc = ensure(&ctx->hhi, z.h_hi, s))) || (z.h_lo && (rc = ensure(&ctx->hlo, z.h_lo, s))) ||
+            (z.gu_part && (rc = ensure(&ctx->gu_part, z.gu_part, s))))
+            return rc;
+    }
     return run_expert(ctx, P, *expert, x, in_dtype, n_tokens, y, out_dtype, y_f32,
                       static_cast<float*>(ctx->hscratch.p), static_cast<uint16_t*>(ctx->hhi.p),
                       static_cast<uint16_t*>(ctx->hlo.p), static_cast<float*>(ctx->gu_part.p), s);
@@ -1309,7 +1298,7 @@ int cx_route(cx_ctx* ctx, const void* x, int x_dtype, const void* w_router, int 
     int rc = fill_route(ctx, x, x_dtype, w_router, w_dtype, bias, resident, n_tokens, hidden,
                         n_experts, n_group, topk_group, top_k, norm_topk_prob,
                         routed_scaling_factor, topk_ids, topk_w, s, &R);
-    if (rc) return rc;
+    if (rc || (rc = route_part(ctx, &R, s))) return rc;
     Span sp(ctx, "route", s);
     CX_HIP(launch_route(R, s));
     return CX_OK;

@@ -1,0 +1,125 @@
+// cx_shapes.h — which kernels a call takes and the scratch it needs, from its
+// sizes alone.  Plain C++, so that the rules can be checked on the host over
+// whole ranges of sizes.
+//
+// A context's scratch only grows, and growing frees the old buffer, which a
+// captured graph may still use.  So what a call asks for covers every call of
+// the same entry point and shape with fewer tokens, whatever kernels these take:
+// a program that has run its largest call allocates no more, under capture too.
+#pragma once
+
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
+
+namespace cx {
+
+// Geometry of the fast grouped kernels.
+constexpr int kKB = 128;        // k-block: one scale per 128 columns
+constexpr int kTileRows = 16;   // MFMA 16x16x32: 16 weight rows per wave
+constexpr int kTileTok = 16;    // 16 token (pair) columns per MFMA tile
+
+constexpr int kDecSplitMaxTokens = 8;  // tokens whose shared gate/up runs as k-parts (8 selection waves)
+
+// ---------------------------------------------------------------------------
+// One expert over 1..4 tokens (split-K down launch).
+constexpr int kDownKsRows = 4;    // tokens
+constexpr int kDownKsGroups = 2;  // 16-row groups per workgroup
+
+inline bool expert_small_shape(int hidden, int inter) {
+    const int nkg = hidden / kKB, nkd = inter / kKB;
+    return hidden % (kDownKsGroups * kTileRows) == 0 && (nkg == 56 || nkg == 8 || nkg == 4) && (nkd == 16 || nkd == 4);
+}
+
+// One expert over 5..64 tokens (single mode, cx_few.h): gate/up writes h in the
+// order the down launch reads it, few_scratch_bytes of it.  The limits, one
+// expert of 7168 x 2048, us a call: 1..4 tokens stay on the k-part launches,
+// whose rows keep their bits whatever the batch (2 tokens 12.4 against 13.3, 4
+// tokens 14.7 against 13.4); 5 tokens 23.7 / 13.5; 64 tokens 31.4 against 41.1
+// with the ping-pong GEMM, 65 tokens 45.4 / 41.3.
+constexpr int kFewMinTokens = 5, kFewMaxTokens = 64;
+constexpr size_t kFewHBlk = 8192;  // h bytes of a 16-token tile and 128 columns: 2 planes x 4 steps x 1 KB
+
+inline int few_tiles(int n_tokens) { return (n_tokens + kTileTok - 1) / kTileTok; }
+
+inline size_t few_scratch_bytes(int n_tokens, int inter) {
+    return (size_t)few_tiles(n_tokens) * (inter / kKB) * kFewHBlk;
+}
+
+inline bool few_ok(int hidden, int inter, int n_tokens) {
+    const int nkg = hidden / kKB, nkd = inter / kKB;
+    return hidden % kKB == 0 && inter % kKB == 0 && (nkg == 56 || nkg == 8 || nkg == 4) && (nkd == 16 || nkd == 4) &&
+           n_tokens >= kFewMinTokens && n_tokens <= kFewMaxTokens;
+}
+
+// Context scratch of a call of cx_expert_run on the fast paths: h as two bf16
+// planes, or all of it in h_hi in fragment order; fp32 k-part sums.
+struct ExpertScratch {
+    size_t h_hi, h_lo, gu_part;
+};
+
+inline ExpertScratch expert_scratch(int n_tokens, int hidden, int inter) {
+    const bool small = expert_small_shape(hidden, inter);
+    const size_t plane = small && n_tokens <= kDownKsRows ? 0 : (size_t)n_tokens * inter * 2;
+    const int few = std::min(n_tokens, kFewMaxTokens);
+    return {std::max(plane, few_ok(hidden, inter, few) ? few_scratch_bytes(few, inter) : 0), plane,
+            small ? sizeof(float) * 2 * 2 * (size_t)std::min(n_tokens, kDownKsRows) * inter : 0};
+}
+
+// ---------------------------------------------------------------------------
+// Router logits of 4 to 256 tokens (k_route_logits_split): K slices, 0: another
+// kernel.
+constexpr int kLsMinTokens = 4, kLsMaxTokens = 256;
+constexpr int kLsWaves = 4;
+constexpr int kLsMaxSlices = 8;
+
+inline int route_slices(int n_tokens, int hidden) {
+    if (n_tokens < kLsMinTokens || n_tokens > kLsMaxTokens || hidden % (kLsWaves * 32) != 0) return 0;
+    int s = n_tokens <= 32 ? 8 : n_tokens <= 64 ? 4 : n_tokens <= 128 ? 2 : 1;
+    while (hidden % (kLsWaves * 32 * s) != 0) s /= 2;
+    return s;
+}
+
+// fp64 cells of the slices: slices x tokens is at most 256 (8 x 32, 4 x 64, 2 x 128).
+constexpr int kLsPartTokens = 256;
+
+inline size_t route_part_cells(int n_tokens, int hidden, int n_experts) {
+    return n_tokens >= kLsMinTokens && hidden % (kLsWaves * 32) == 0 ? (size_t)kLsPartTokens * n_experts : 0;
+}
+
+// ---------------------------------------------------------------------------
+// The plan of a grouped call (PlanPtrs).
+constexpr int kPlanHdrInts = 8;
+constexpr size_t kItemRecBytes = 88, kSlotRecBytes = 24;
+
+struct PlanSizes {
+    int max_slots, max_pairs, max_items, item_cap, maxt;
+};
+
+inline PlanSizes plan_sizes(int n_tokens, int top_k, int n_experts, int has_shared) {
+    PlanSizes z;
+    z.maxt = n_tokens <= kTileTok ? 1 : 4;
+    z.item_cap = kTileTok * z.maxt;
+    z.max_slots = std::min(n_tokens * top_k, n_experts) + has_shared;
+    z.max_pairs = n_tokens * top_k + n_tokens * has_shared;
+    z.max_items = z.max_slots + (z.max_pairs + z.item_cap - 1) / z.item_cap;
+    return z;
+}
+
+// dense: a decode plan, which also fills pair_row.
+inline size_t plan_bytes(const PlanSizes& z, int n_tokens, int top_k, bool dense) {
+    const size_t ints = kPlanHdrInts + 3 * (size_t)z.max_slots + 3 * (size_t)z.max_items +
+                        2 * (size_t)z.max_pairs + (size_t)n_tokens * (top_k + 1) +
+                        (dense ? (size_t)z.max_pairs : 0);
+    return kItemRecBytes * (size_t)z.max_items + kSlotRecBytes * (size_t)z.max_slots + ints * 4;
+}
+
+// Bytes of the plan buffer: the plan with the smallest items (16 pairs) and
+// pair_row, so that neither the item size nor the pipeline makes it shrink.
+inline size_t plan_buffer_bytes(int n_tokens, int top_k, int n_experts, int has_shared) {
+    PlanSizes z = plan_sizes(n_tokens, top_k, n_experts, has_shared);
+    z.max_items = z.max_slots + (z.max_pairs + kTileTok - 1) / kTileTok;
+    return plan_bytes(z, n_tokens, top_k, true);
+}
+
+}  // namespace cx

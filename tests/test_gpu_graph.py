@@ -73,3 +73,68 @@ def test_moe_layer_graph_replays_equal_eager(gpu, T):
         for e in experts:
             e.free()
         sh.free()
+
+
+def _smaller_calls(gpu, kind, H, I, E):
+    """(tokens of the largest call, smaller ones, call(T, context) -> outputs, cleanup)."""
+    from constellation_amd.engine import Expert, Layer
+    x = gpu.gen_normal(131, 1, (700, H), 1.0, torch.bfloat16)
+    w_r = gpu.gen_normal(131, 2, (E, H), 0.02, torch.bfloat16)
+    bias = gpu.gen_normal(131, 3, (E,), 0.01, torch.float32)
+    opt = dict(n_group=8, topk_group=4, top_k=8)
+    if kind == "route":
+        return 256, (128, 64, 32, 5, 1), lambda T, c: c.route(x[:T], w_r, bias, **opt), lambda: None
+    if kind == "expert":
+        e = Expert.generate(0, 132, 0x2800, hidden=H, inter=I)
+        return 90, (65, 64, 33, 16, 5, 2), lambda T, c: (c.expert_run(e, x[:T]),), e.free
+    experts = [Expert.generate(0, 132, 0x2800 + 4 * e, hidden=H, inter=I) for e in range(E + 1)]
+    layer = Layer(gpu, experts[:E], experts[E])
+
+    def free():
+        layer.close()
+        for e in experts:
+            e.free()
+
+    def call(T, c):
+        y, _, ids, w = c.moe_layer(layer, x[:T], w_r, bias, **opt)
+        return y, ids, w
+    return 161, (160, 159, 100, 40, 17, 16, 8, 1), call, free
+
+
+@pytest.mark.parametrize("kind", ["route", "expert", "layer"])
+def test_smaller_calls_need_no_more_scratch(gpu, kind):
+    """After one eager call, every smaller call of the same shape is captured
+    without an eager one of its own (a capture in which scratch grows fails),
+    whichever kernels it takes; then the captured graphs are replayed with
+    eager calls of all these sizes between them, twice, and still equal
+    another context's results: none of them moved the scratch of another."""
+    from constellation_amd.engine import Context
+    print(f"[graph] smaller calls, {kind}", flush=True)
+    most, sizes, call, free = _smaller_calls(gpu, kind, 1024, 512, 64)
+    graphs = {}
+    try:
+        with Context(0) as ctx:
+            side = torch.cuda.Stream()
+            with torch.cuda.stream(side):
+                call(most, ctx)
+            torch.cuda.synchronize()
+            for T in sizes:
+                g = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(g, stream=side, capture_error_mode="thread_local"):
+                    graphs[T] = (g, call(T, ctx))
+                torch.cuda.synchronize()
+            for _ in range(2):
+                for T, (g, got) in graphs.items():
+                    for t in sizes:
+                        call(t, ctx)
+                    torch.cuda.synchronize()
+                    g.replay()
+                    torch.cuda.synchronize()
+                    want = call(T, gpu)
+                    torch.cuda.synchronize()
+                    assert all(torch.equal(a, b) for a, b in zip(got, want)), T
+            torch.cuda.synchronize()
+            graphs.clear()
+    finally:
+        torch.cuda.synchronize()
+        free()

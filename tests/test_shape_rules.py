@@ -1,0 +1,82 @@
+"""The rules of csrc/cx_shapes.h over ranges of sizes, on the host: the scratch a
+call asks for covers what its kernels use and every call with fewer tokens."""
+from __future__ import annotations
+
+import ctypes as C
+import subprocess
+from pathlib import Path
+
+import pytest
+
+CSRC = Path(__file__).resolve().parent.parent / "constellation_amd" / "csrc"
+
+SOURCE = r"""
+#include "cx_shapes.h"
+using namespace cx;
+extern "C" {
+void expert(int t, int h, int i, size_t* out) {
+    const ExpertScratch z = expert_scratch(t, h, i);
+    out[0] = z.h_hi; out[1] = z.h_lo; out[2] = z.gu_part;
+}
+int small(int h, int i) { return expert_small_shape(h, i); }
+size_t few_bytes(int t, int i) { return few_scratch_bytes(t, i); }
+int few(int h, int i, int t) { return few_ok(h, i, t); }
+int slices(int t, int h) { return route_slices(t, h); }
+size_t part(int t, int h, int e) { return route_part_cells(t, h, e); }
+size_t buffer(int t, int k, int e, int sh) { return plan_buffer_bytes(t, k, e, sh); }
+size_t plan(int t, int k, int e, int sh, int cap, int dense) {
+    PlanSizes z = plan_sizes(t, k, e, sh);
+    z.max_items = dense ? z.max_slots : z.max_slots + (z.max_pairs + cap - 1) / cap;
+    return plan_bytes(z, t, k, dense);
+}
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.cc").write_text(SOURCE)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}",
+                    str(d / "rules.cc"), "-o", str(d / "rules.so")], check=True)
+    L = C.CDLL(str(d / "rules.so"))
+    for f in ("few_bytes", "part", "buffer", "plan"):
+        getattr(L, f).restype = C.c_size_t
+    return L
+
+
+@pytest.mark.parametrize("H,I", [(7168, 2048), (1024, 512), (512, 512), (7168, 512), (4096, 1536), (2048, 768)])
+def test_expert_scratch_never_shrinks(rules, H, I):
+    last = (0, 0, 0)
+    for T in range(1, 700):
+        out = (C.c_size_t * 3)()
+        rules.expert(T, H, I, out)
+        got = tuple(out)
+        assert all(a <= b for a, b in zip(last, got)), (T, last, got)
+        last = got
+        if T <= 4 and rules.small(H, I):
+            need = (0, 0, 16 * T * I)  # two k-parts of gate and up, fp32
+        else:
+            need = (max(2 * T * I, rules.few_bytes(T, I) if rules.few(H, I, T) else 0), 2 * T * I, 0)
+        assert all(n <= b for n, b in zip(need, got)), (T, need, got)
+
+
+@pytest.mark.parametrize("H,E", [(7168, 256), (1024, 64), (640, 72), (384, 40), (1000, 8)])
+def test_router_slices_never_shrink(rules, H, E):
+    last = 0
+    for T in range(1, 600):
+        got = rules.part(T, H, E)
+        assert got >= last and got >= rules.slices(T, H) * T * E, T
+        last = got
+
+
+@pytest.mark.parametrize("E,K", [(256, 8), (64, 8), (4, 2), (128, 1), (512, 64)])
+@pytest.mark.parametrize("shared", [0, 1])
+def test_plan_buffer_never_shrinks(rules, E, K, shared):
+    last = 0
+    for T in range(1, 1500):
+        got = rules.buffer(T, K, E, shared)
+        assert got >= last, T
+        last = got
+        forms = [(64, 0), (128, 0)] if T > 16 else [(16, 0), (16, 1), (128, 0)]
+        assert all(rules.plan(T, K, E, shared, cap, dense) <= got for cap, dense in forms), T
