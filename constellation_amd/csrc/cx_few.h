@@ -27,7 +27,6 @@
 namespace cx {
 
 constexpr int kFewGuRows = 8;    // outputs per gate/up workgroup
-constexpr int kFewGuWaves = 8;
 constexpr int kFewDnRows = 32;
 constexpr int kFewDnWaves = 4;
 
@@ -37,7 +36,6 @@ constexpr int kFewDnWaves = 4;
 // fragments through the wave's own LDS, chunk q of token t at q ^ t: loaded
 // straight into fragment order, 16 tokens x 64 B an instruction, one expert's
 // gate/up took 8.6 / 12.7 / 29 us at 1 / 16 / 64 tokens.
-constexpr int few_gu_lds(int nt) { return kFewGuWaves * nt * 4096; }
 
 template <int NKB, int KSA, int NT, int D, bool F16>
 __device__ __forceinline__ void few_gate_up(const ExpertLaunch& L, unsigned char* lds) {

@@ -43,7 +43,7 @@ void go_dn(const ExpertLaunch& L, hipStream_t s) {
 }  // namespace
 
 hipError_t launch_gate_up_few(const ExpertLaunch& L, hipStream_t s) {
-    if (L.table != nullptr || !few_ok(L.hidden, L.inter, L.n_tokens)) return hipErrorInvalidValue;
+    if (L.table != nullptr || !few_ok(L.hidden, L.inter, L.n_tokens, L.max_lds)) return hipErrorInvalidValue;
     const bool f16 = L.in_dtype == CX_DTYPE_FP16;
     switch (few_tiles(L.n_tokens)) {
         case 1: f16 ? pick_gu<1, true>(L, s) : pick_gu<1, false>(L, s); break;
@@ -55,7 +55,7 @@ hipError_t launch_gate_up_few(const ExpertLaunch& L, hipStream_t s) {
 }
 
 hipError_t launch_down_few(const ExpertLaunch& L, hipStream_t s) {
-    if (L.table != nullptr || !few_ok(L.hidden, L.inter, L.n_tokens)) return hipErrorInvalidValue;
+    if (L.table != nullptr || !few_ok(L.hidden, L.inter, L.n_tokens, L.max_lds)) return hipErrorInvalidValue;
     const bool full = L.inter / kKB == 16;
     switch (few_tiles(L.n_tokens)) {
         case 1: full ? go_dn<4, 1>(L, s) : go_dn<1, 1>(L, s); break;

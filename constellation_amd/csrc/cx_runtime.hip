@@ -410,7 +410,7 @@ ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int
     L.np_lds = L.maxt == 1 ? lds_rows(max_lds, e.hidden, n_tokens) : 0;
     L.max_lds = max_lds;
     L.n_cu = n_cu;
-    if (few_ok(e.hidden, e.inter, n_tokens)) {
+    if (few_ok(e.hidden, e.inter, n_tokens, max_lds)) {
         P.path = kPathFew;
         P.h_frag_bytes = few_scratch_bytes(n_tokens, e.inter);
     } else if (expert_small_ok(L)) {
@@ -1153,7 +1153,7 @@ int cx_expert_run(cx_ctx* ctx, const cx_expert_desc* expert, const void* x, int 
     ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->max_lds, ctx->n_cu);
     if (P.h_f32_bytes && (rc = ensure(&ctx->hscratch, P.h_f32_bytes, s))) return rc;
     if (P.path != kPathGeneric) {
-        const ExpertScratch z = expert_scratch(n_tokens, expert->hidden, expert->inter);
+        const ExpertScratch z = expert_scratch(n_tokens, expert->hidden, expert->inter, ctx->max_lds);
         if ((z.h_hi && (rc = ensure(&ctx->hhi, z.h_hi, s))) || (z.h_lo && (rc = ensure(&ctx->hlo, z.h_lo, s))) ||
             (z.gu_part && (rc = ensure(&ctx->gu_part, z.gu_part, s))))
             return rc;

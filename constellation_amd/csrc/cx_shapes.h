@@ -39,17 +39,24 @@ inline bool expert_small_shape(int hidden, int inter) {
 // with the ping-pong GEMM, 65 tokens 45.4 / 41.3.
 constexpr int kFewMinTokens = 5, kFewMaxTokens = 64;
 constexpr size_t kFewHBlk = 8192;  // h bytes of a 16-token tile and 128 columns: 2 planes x 4 steps x 1 KB
+constexpr int kFewGuWaves = 8;     // waves of a gate/up workgroup
+
+// LDS of a gate/up workgroup: a block of x, later a partial tile, per wave and tile.
+constexpr int few_gu_lds(int tiles) { return kFewGuWaves * tiles * 4096; }
 
 inline int few_tiles(int n_tokens) { return (n_tokens + kTileTok - 1) / kTileTok; }
+
+// The most tokens whose LDS a workgroup of this device can have (32 with 64 KB).
+inline int few_max_tokens(int max_lds) { return std::min(kFewMaxTokens, max_lds / few_gu_lds(1) * kTileTok); }
 
 inline size_t few_scratch_bytes(int n_tokens, int inter) {
     return (size_t)few_tiles(n_tokens) * (inter / kKB) * kFewHBlk;
 }
 
-inline bool few_ok(int hidden, int inter, int n_tokens) {
+inline bool few_ok(int hidden, int inter, int n_tokens, int max_lds) {
     const int nkg = hidden / kKB, nkd = inter / kKB;
     return hidden % kKB == 0 && inter % kKB == 0 && (nkg == 56 || nkg == 8 || nkg == 4) && (nkd == 16 || nkd == 4) &&
-           n_tokens >= kFewMinTokens && n_tokens <= kFewMaxTokens;
+           n_tokens >= kFewMinTokens && n_tokens <= few_max_tokens(max_lds);
 }
 
 // Context scratch of a call of cx_expert_run on the fast paths: h as two bf16
@@ -58,11 +65,11 @@ struct ExpertScratch {
     size_t h_hi, h_lo, gu_part;
 };
 
-inline ExpertScratch expert_scratch(int n_tokens, int hidden, int inter) {
+inline ExpertScratch expert_scratch(int n_tokens, int hidden, int inter, int max_lds) {
     const bool small = expert_small_shape(hidden, inter);
     const size_t plane = small && n_tokens <= kDownKsRows ? 0 : (size_t)n_tokens * inter * 2;
-    const int few = std::min(n_tokens, kFewMaxTokens);
-    return {std::max(plane, few_ok(hidden, inter, few) ? few_scratch_bytes(few, inter) : 0), plane,
+    const int few = std::min(n_tokens, few_max_tokens(max_lds));
+    return {std::max(plane, few_ok(hidden, inter, few, max_lds) ? few_scratch_bytes(few, inter) : 0), plane,
             small ? sizeof(float) * 2 * 2 * (size_t)std::min(n_tokens, kDownKsRows) * inter : 0};
 }
 

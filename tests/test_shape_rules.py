@@ -14,13 +14,14 @@ SOURCE = r"""
 #include "cx_shapes.h"
 using namespace cx;
 extern "C" {
-void expert(int t, int h, int i, size_t* out) {
-    const ExpertScratch z = expert_scratch(t, h, i);
+void expert(int t, int h, int i, int lds, size_t* out) {
+    const ExpertScratch z = expert_scratch(t, h, i, lds);
     out[0] = z.h_hi; out[1] = z.h_lo; out[2] = z.gu_part;
 }
 int small(int h, int i) { return expert_small_shape(h, i); }
 size_t few_bytes(int t, int i) { return few_scratch_bytes(t, i); }
-int few(int h, int i, int t) { return few_ok(h, i, t); }
+int few(int h, int i, int t, int lds) { return few_ok(h, i, t, lds); }
+int few_lds(int t) { return few_gu_lds(few_tiles(t)); }
 int slices(int t, int h) { return route_slices(t, h); }
 size_t part(int t, int h, int e) { return route_part_cells(t, h, e); }
 size_t buffer(int t, int k, int e, int sh) { return plan_buffer_bytes(t, k, e, sh); }
@@ -45,20 +46,28 @@ def rules(tmp_path_factory):
     return L
 
 
+@pytest.mark.parametrize("lds", [160 << 10, 64 << 10])
 @pytest.mark.parametrize("H,I", [(7168, 2048), (1024, 512), (512, 512), (7168, 512), (4096, 1536), (2048, 768)])
-def test_expert_scratch_never_shrinks(rules, H, I):
+def test_expert_scratch_never_shrinks(rules, H, I, lds):
     last = (0, 0, 0)
     for T in range(1, 700):
         out = (C.c_size_t * 3)()
-        rules.expert(T, H, I, out)
+        rules.expert(T, H, I, lds, out)
         got = tuple(out)
         assert all(a <= b for a, b in zip(last, got)), (T, last, got)
         last = got
         if T <= 4 and rules.small(H, I):
             need = (0, 0, 16 * T * I)  # two k-parts of gate and up, fp32
         else:
-            need = (max(2 * T * I, rules.few_bytes(T, I) if rules.few(H, I, T) else 0), 2 * T * I, 0)
+            need = (max(2 * T * I, rules.few_bytes(T, I) if rules.few(H, I, T, lds) else 0), 2 * T * I, 0)
         assert all(n <= b for n, b in zip(need, got)), (T, need, got)
+
+
+@pytest.mark.parametrize("lds", [160 << 10, 96 << 10, 64 << 10, 16 << 10])
+def test_few_token_kernels_fit_the_lds(rules, lds):
+    """5..64 tokens where a workgroup can have the LDS, else the other kernels."""
+    for T in range(1, 80):
+        assert bool(rules.few(7168, 2048, T, lds)) == (5 <= T <= 64 and rules.few_lds(T) <= lds), T
 
 
 @pytest.mark.parametrize("H,E", [(7168, 256), (1024, 64), (640, 72), (384, 40), (1000, 8)])
