@@ -171,7 +171,7 @@ struct ExpertLaunch {
     float* y_f32;                 // single mode / fused decode: optional fp32 output
     int out_dtype;
     int fold_weight;              // phase A multiplies h by the pair's route weight
-    int np_lds;                   // >0: stage up to np_lds activation rows per item in LDS
+    int np_lds;                   // >0: stage up to np_lds activation rows (x dma_aligned) per item in LDS
     int skip_shared;              // grouped mode: routed items only (shared expert done apart)
     int max_lds;                  // dynamic LDS per workgroup the device allows (0: unknown)
     float* gu_part;               // k-part gate/up sums of the shared expert [kparts][2][T][inter]
@@ -183,9 +183,8 @@ struct ExpertLaunch {
 hipError_t launch_gate_up(const ExpertLaunch& L, hipStream_t s);
 // The ping-pong GEMM (cx_pp.h): grouped mode with items of up to kBigPairs (128)
 // pairs, for calls with many tokens per expert, and single mode; gate/up writes
-// h, down writes y_part or the output, as launch_gate_up / launch_down do.
-// pp_ok: the shapes they take.
-bool pp_ok(int hidden, int inter, int max_lds);
+// h, down writes y_part or the output, as launch_gate_up / launch_down do, for the
+// shapes of pp_ok.  x and the weights must be dma_aligned.
 hipError_t launch_gate_up_pp(const ExpertLaunch& L, hipStream_t s);
 hipError_t launch_down_pp(const ExpertLaunch& L, hipStream_t s);
 // Down projection per work item: grouped mode writes fp32 y_part[pair]
@@ -214,7 +213,8 @@ hipError_t launch_plan(const int32_t* ids, const float* w, int n_tokens, int top
                        int item_cap, int max_items, PlanPtrs plan, int* err_flag,
                        hipStream_t s);
 
-// One expert over 5..64 tokens (few_ok): h in fragment order from L.h_hi on.
+// One expert over 5..64 tokens (few_ok): h in fragment order from L.h_hi on.  x
+// must be dma_aligned.
 hipError_t launch_gate_up_few(const ExpertLaunch& L, hipStream_t s);
 hipError_t launch_down_few(const ExpertLaunch& L, hipStream_t s);
 

@@ -14,14 +14,10 @@
 
 namespace cx {
 
-constexpr int kPpRowsGu = 128;  // inter rows (of gate and of up) per gate/up workgroup
-constexpr int kPpRowsDn = 256;  // hidden rows per down workgroup
 constexpr int kPpK = 64;        // k of half a 128-column scale block
 constexpr int kPpA = 16384;     // weight bytes of a half block: 16 tiles x 16 rows x 64 k
 constexpr int kPpTile = 2048;   // activation bytes of a 16-pair column tile and plane in a half block
-constexpr int kPpMinBlocks = 4;  // 128-column blocks of a row: the ring's last blocks are peeled off
 constexpr int kPpMaxTiles = kBigPairs / kTileTok;
-constexpr int kPpLds = 160 * 1024;  // one workgroup per CU
 
 // Weight tiles per wave.  The down projection of more than four column tiles
 // splits the columns over the two waves of a SIMD (see pp_core), which computes

@@ -49,11 +49,6 @@ dim3 pp_grid(const ExpertLaunch& L, int row_tiles) {
 
 }  // namespace
 
-bool pp_ok(int hidden, int inter, int max_lds) {
-    return inter % kPpRowsGu == 0 && hidden % kPpRowsDn == 0 && hidden / kKB >= kPpMinBlocks &&
-           inter / kKB >= kPpMinBlocks && max_lds >= kPpLds;
-}
-
 hipError_t launch_gate_up_pp(const ExpertLaunch& L0, hipStream_t s) {
     ExpertLaunch L = L0;
     if (!pp_ok(L.hidden, L.inter, L.max_lds)) return hipErrorInvalidValue;

@@ -261,6 +261,7 @@ struct cx_layer {
     cx_expert_desc shared_desc{};      // host copy of the shared expert (when has_shared)
     std::vector<uint8_t> resident;     // host copy: entry i holds an expert
     int n_resident = 0;                // routed experts held
+    bool dma = true;                   // every weight matrix is dma_aligned
 };
 
 namespace {
@@ -357,29 +358,14 @@ int check_desc(const cx_expert_desc* e) {
     return CX_OK;
 }
 
-// Activation rows of one work item that fit the LDS budget next to the
-// reduction tile (<= 16 KB); 0 when staging is not worth it or not possible.
-int lds_rows(int max_lds, int hidden, int max_pairs_per_item) {
-    if (hidden % 512 != 0) return 0;  // rows are copied in 1 KB wave chunks
-    const int budget = std::min(max_lds, 65536) - 16384;
-    const int rows = budget / (hidden * 2 + 16);
-    return (max_pairs_per_item <= rows && max_pairs_per_item <= 4) ? max_pairs_per_item : 0;
-}
-
-int lds_rows(const cx_ctx* ctx, int hidden, int max_pairs_per_item) {
-    return lds_rows(ctx->max_lds, hidden, max_pairs_per_item);
-}
-
 // ---------------------------------------------------------------------------
 // One expert over n_tokens tokens (single mode: the tokens are the pairs, the
 // down launch writes the output).  Shared by cx_expert_run (context scratch)
 // and cx_expert_run_static (the library's static device scratch): plan_expert
 // picks the path and states the scratch it needs, run_expert launches it.
-enum ExpertPath { kPathGeneric, kPathSmall, kPathTiles, kPathPingPong, kPathFew };
-
 struct ExpertPlan {
     ExpertLaunch L;
-    int path;
+    ExpertRoute route;
     size_t h_f32_bytes;   // generic path: fp32 h [T, I]
     size_t h_plane_bytes; // tile paths: each bf16 plane h_hi / h_lo [T, I]
     size_t h_frag_bytes;  // few-token path: h in fragment order
@@ -391,7 +377,7 @@ ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int
     ExpertPlan P{};
     const size_t TI = (size_t)n_tokens * e.inter;
     if (!fast_path_ok(e)) {
-        P.path = kPathGeneric;
+        P.route.path = kPathGeneric;
         P.h_f32_bytes = TI * 4;
         return P;
     }
@@ -407,21 +393,17 @@ ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int
     L.y = y;
     L.y_f32 = y_f32;
     L.out_dtype = out_dtype;
-    L.np_lds = L.maxt == 1 ? lds_rows(max_lds, e.hidden, n_tokens) : 0;
     L.max_lds = max_lds;
     L.n_cu = n_cu;
-    if (few_ok(e.hidden, e.inter, n_tokens, max_lds)) {
-        P.path = kPathFew;
+    P.route = expert_route(n_tokens, e.hidden, e.inter, max_lds, dma_aligned(x),
+                           dma_aligned(e.w_gate) && dma_aligned(e.w_up), dma_aligned(e.w_down));
+    L.np_lds = P.route.np_lds;
+    if (P.route.path == kPathFew) {
         P.h_frag_bytes = few_scratch_bytes(n_tokens, e.inter);
-    } else if (expert_small_ok(L)) {
-        P.path = kPathSmall;
+    } else if (P.route.path == kPathSmall) {
         P.gu_part_bytes = sizeof(float) * 2 * 2 * TI;
         L.gu_kparts = 2;
     } else {
-        // above 16 tokens the 64-token items of the grouped kernels leave most
-        // CUs idle (16 gate/up workgroups at 17..64 tokens): 66 / 108 us at 32 /
-        // 300 tokens against 42 / 59 with the ping-pong GEMM
-        P.path = L.maxt > 1 && pp_ok(e.hidden, e.inter, max_lds) ? kPathPingPong : kPathTiles;
         P.h_plane_bytes = TI * 2;
     }
     return P;
@@ -433,12 +415,12 @@ ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int
 int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* x, int in_dtype,
                int n_tokens, void* y, int out_dtype, float* y_f32, float* h_f32, uint16_t* h_hi,
                uint16_t* h_lo, float* gu_part, hipStream_t s) {
-    if (P.path == kPathGeneric) {
+    if (P.route.path == kPathGeneric) {
         CX_HIP(launch_generic_expert(e, x, in_dtype, n_tokens, h_f32, y, out_dtype, y_f32, s));
         return CX_OK;
     }
     ExpertLaunch& L = P.L;
-    if (P.path == kPathSmall) {
+    if (P.route.path == kPathSmall) {
         L.gu_part = gu_part;
         {
             Span sp(ctx, "gate_up", s);
@@ -450,7 +432,7 @@ int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* 
     }
     L.h_hi = h_hi;
     L.h_lo = h_lo;
-    if (P.path == kPathFew) {
+    if (P.route.path == kPathFew) {
         {
             Span sp(ctx, "gate_up", s);
             CX_HIP(launch_gate_up_few(L, s));
@@ -461,11 +443,11 @@ int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* 
     }
     {
         Span sp(ctx, "gate_up", s);
-        CX_HIP(P.path == kPathPingPong ? launch_gate_up_pp(L, s) : launch_gate_up(L, s));
+        CX_HIP(P.route.pp_gate_up ? launch_gate_up_pp(L, s) : launch_gate_up(L, s));
     }
     {
         Span sp(ctx, "down", s);
-        CX_HIP(P.path == kPathPingPong ? launch_down_pp(L, s) : launch_down(L, s));
+        CX_HIP(P.route.pp_down ? launch_down_pp(L, s) : launch_down(L, s));
     }
     return CX_OK;
 }
@@ -543,7 +525,8 @@ int moe_decode(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, 
                float* y_f32, hipStream_t s, RouteArgs* route, const PlanSizes& z,
                const PlanPtrs& P) {
     const int T = n_tokens;
-    const int np_lds = lds_rows(ctx, layer->hidden, T);
+    const bool x_dma = dma_aligned(x);
+    const int np_lds = lds_rows(ctx->max_lds, layer->hidden, T, x_dma);
     ExpertLaunch SG{};
     SG.table = nullptr;
     SG.single = layer->shared_desc;
@@ -556,7 +539,7 @@ int moe_decode(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, 
     SG.h_hi = static_cast<uint16_t*>(ctx->hhi.p);  // shared pairs [0, T)
     SG.h_lo = static_cast<uint16_t*>(ctx->hlo.p);
     SG.y_part = static_cast<float*>(ctx->ypart.p);
-    SG.np_lds = route != nullptr ? dec_sgu_np_lds(layer->hidden, T, ctx->max_lds) : 0;
+    SG.np_lds = route != nullptr && x_dma ? dec_sgu_np_lds(layer->hidden, T, ctx->max_lds) : 0;
     const ExpertLaunch* sg = layer->has_shared ? &SG : nullptr;
     // T <= 8 with the router: the shared gate/up tiles run as two k-parts
     // (twice the CUs); the routed gate/up launch finalises the shared h
@@ -699,7 +682,8 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
     // route tables masked to one node of several (-1 for other nodes' experts)
     // can then take it with mostly-padding tiles (correct, slower).
     const int64_t pairs = valid_routes >= 0 ? valid_routes : (int64_t)n_tokens * top_k;
-    const bool big = !dec && pp_ok(layer->hidden, layer->inter, ctx->max_lds) &&
+    const bool x_dma = dma_aligned(x);
+    const bool big = !dec && x_dma && layer->dma && pp_ok(layer->hidden, layer->inter, ctx->max_lds) &&
                      pairs >= (int64_t)kBigMinPairs * std::max(1, layer->n_resident);
     if (big) {
         z.item_cap = kBigPairs;
@@ -752,7 +736,7 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
     L.y = y;
     L.y_f32 = y_f32;
     L.out_dtype = out_dtype;
-    L.np_lds = z.maxt == 1 ? lds_rows(ctx, layer->hidden, std::min(n_tokens, z.item_cap)) : 0;
+    L.np_lds = z.maxt == 1 ? lds_rows(ctx->max_lds, layer->hidden, std::min(n_tokens, z.item_cap), x_dma) : 0;
     L.max_lds = ctx->max_lds;
     {
         Span sp(ctx, "gate_up", s);
@@ -1152,7 +1136,7 @@ int cx_expert_run(cx_ctx* ctx, const cx_expert_desc* expert, const void* x, int 
     hipStream_t s = static_cast<hipStream_t>(stream);
     ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->max_lds, ctx->n_cu);
     if (P.h_f32_bytes && (rc = ensure(&ctx->hscratch, P.h_f32_bytes, s))) return rc;
-    if (P.path != kPathGeneric) {
+    if (P.route.path != kPathGeneric) {
         const ExpertScratch z = expert_scratch(n_tokens, expert->hidden, expert->inter, ctx->max_lds);
         if ((z.h_hi && (rc = ensure(&ctx->hhi, z.h_hi, s))) || (z.h_lo && (rc = ensure(&ctx->hlo, z.h_lo, s))) ||
             (z.gu_part && (rc = ensure(&ctx->gu_part, z.gu_part, s))))
@@ -1242,6 +1226,7 @@ int cx_layer_create(cx_ctx* ctx, int n_experts, const cx_expert_desc* const* exp
     std::vector<cx_expert_desc> host(n_experts + 1);
     std::memset(host.data(), 0, sizeof(cx_expert_desc) * host.size());
     int H = 0, I = 0, fast = 1, any = 0;
+    bool dma = true;
     auto take = [&](const cx_expert_desc* e, cx_expert_desc* dst) -> int {
         int r = check_desc(e);
         if (r) return r;
@@ -1251,6 +1236,7 @@ int cx_layer_create(cx_ctx* ctx, int n_experts, const cx_expert_desc* const* exp
         I = e->inter;
         any = 1;
         fast &= fast_path_ok(*e) ? 1 : 0;
+        dma = dma && dma_aligned(e->w_gate) && dma_aligned(e->w_up) && dma_aligned(e->w_down);
         *dst = *e;
         return CX_OK;
     };
@@ -1267,6 +1253,7 @@ int cx_layer_create(cx_ctx* ctx, int n_experts, const cx_expert_desc* const* exp
     for (int i = 0; i < n_experts; ++i) L->n_resident += L->resident[i];
     L->shared_desc = host[n_experts];
     L->fast = fast;
+    L->dma = dma;
     L->hidden = H;
     L->inter = I;
     if (hipMalloc(&L->table, sizeof(cx_expert_desc) * host.size()) != hipSuccess ||

@@ -21,6 +21,21 @@ constexpr int kTileTok = 16;    // 16 token (pair) columns per MFMA tile
 
 constexpr int kDecSplitMaxTokens = 8;  // tokens whose shared gate/up runs as k-parts (8 selection waves)
 
+// The ABI states no alignment of x, and a view's rows may start anywhere.  Direct
+// global->LDS loads and bounded buffer loads, 16 bytes a lane, are only given rows
+// (and weights) that start on 16 bytes; all others go through plain loads, which
+// take any address.
+inline bool dma_aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// Activation rows of one work item that fit the LDS budget next to the
+// reduction tile (<= 16 KB); 0 when staging is not worth it or not possible.
+inline int lds_rows(int max_lds, int hidden, int max_pairs_per_item, bool x_dma) {
+    if (!x_dma || hidden % 512 != 0) return 0;  // rows are copied in 1 KB wave chunks
+    const int budget = std::min(max_lds, 65536) - 16384;
+    const int rows = budget / (hidden * 2 + 16);
+    return (max_pairs_per_item <= rows && max_pairs_per_item <= 4) ? max_pairs_per_item : 0;
+}
+
 // ---------------------------------------------------------------------------
 // One expert over 1..4 tokens (split-K down launch).
 constexpr int kDownKsRows = 4;    // tokens
@@ -57,6 +72,42 @@ inline bool few_ok(int hidden, int inter, int n_tokens, int max_lds) {
     const int nkg = hidden / kKB, nkd = inter / kKB;
     return hidden % kKB == 0 && inter % kKB == 0 && (nkg == 56 || nkg == 8 || nkg == 4) && (nkd == 16 || nkd == 4) &&
            n_tokens >= kFewMinTokens && n_tokens <= few_max_tokens(max_lds);
+}
+
+// The ping-pong GEMM (cx_pp.h).
+constexpr int kPpRowsGu = 128;  // inter rows (of gate and of up) per gate/up workgroup
+constexpr int kPpRowsDn = 256;  // hidden rows per down workgroup
+constexpr int kPpMinBlocks = 4;  // 128-column blocks of a row: the ring's last blocks are peeled off
+constexpr int kPpLds = 160 * 1024;  // one workgroup per CU
+
+inline bool pp_ok(int hidden, int inter, int max_lds) {
+    return inter % kPpRowsGu == 0 && hidden % kPpRowsDn == 0 && hidden / kKB >= kPpMinBlocks &&
+           inter / kKB >= kPpMinBlocks && max_lds >= kPpLds;
+}
+
+// Kernels of one expert on the fast paths.  Above 16 tokens the 64-token items of
+// the grouped kernels leave most CUs idle (16 gate/up workgroups at 17..64
+// tokens): 66 / 108 us at 32 / 300 tokens against 42 / 59 with the ping-pong GEMM.
+// x_dma, gu_dma, down_dma: x, the gate and up and the down weights are dma_aligned.
+enum ExpertPath { kPathGeneric, kPathSmall, kPathTiles, kPathFew };
+
+struct ExpertRoute {
+    ExpertPath path;
+    bool pp_gate_up, pp_down;  // kPathTiles: this launch by the ping-pong GEMM
+    int np_lds;                // rows of x staged in LDS
+};
+
+inline ExpertRoute expert_route(int n_tokens, int hidden, int inter, int max_lds, bool x_dma, bool gu_dma, bool down_dma) {
+    ExpertRoute r{kPathTiles, false, false, n_tokens <= kTileTok ? lds_rows(max_lds, hidden, n_tokens, x_dma) : 0};
+    if (x_dma && few_ok(hidden, inter, n_tokens, max_lds)) {
+        r.path = kPathFew;
+    } else if (n_tokens <= kDownKsRows && expert_small_shape(hidden, inter)) {
+        r.path = kPathSmall;
+    } else if (n_tokens > kTileTok && pp_ok(hidden, inter, max_lds)) {
+        r.pp_gate_up = x_dma && gu_dma;
+        r.pp_down = down_dma;
+    }
+    return r;
 }
 
 // Context scratch of a call of cx_expert_run on the fast paths: h as two bf16

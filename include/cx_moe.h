@@ -161,7 +161,10 @@ CX_API int cx_ctx_profile_read(cx_ctx* ctx, const char* kernel, int* launches,
  * Semantics of RunExpertCudaV2 (backend/cuda/backend_cuda_v2.cc:205-255)
  * and RunExpertReferenceV2 (backend/expert_reference_v2.cc:146-178), with
  * batch >= 1 instead of the reference's batch == 1
- * (backend_workspace_cuda_v2.cc:146) and both fp16 and bf16 in/out. */
+ * (backend_workspace_cuda_v2.cc:146) and both fp16 and bf16 in/out.
+ * x, here and in the entry points below, may start at any address; the kernels
+ * with direct global->LDS loads take it where it starts on 16 bytes, slower
+ * ones with plain loads otherwise. */
 CX_API int cx_expert_run(cx_ctx* ctx, const cx_expert_desc* expert,
                   const void* x, int in_dtype, int n_tokens,
                   void* y, int out_dtype, float* y_f32, void* stream);

@@ -301,6 +301,32 @@ def test_few_tokens_one_expert(gpu, oracle, H, I, Ts, dt, tiled):
         e.free()
 
 
+@pytest.mark.parametrize("off", [1, 4])
+@pytest.mark.parametrize("H,I,dt", [(1024, 512, BF16), (512, 512, FP16), (7168, 2048, BF16)])
+def test_rows_that_start_between_16_bytes(gpu, H, I, dt, off):
+    """x of any address: a view that starts 2 or 8 bytes past a 16-byte boundary
+    takes the kernels with plain loads, for every count of tokens that else takes
+    wider ones (in LDS, few-token, ping-pong), and equals its aligned copy."""
+    from constellation_amd.engine import Expert
+    e = Expert.generate(0, 97, 0x7c0, hidden=H, inter=I)
+    try:
+        for T in (1, 3, 5, 16, 17, 64, 65, 200):
+            print(f"[expert] x at +{2 * off} bytes H={H} T={T}", flush=True)
+            x = gpu.gen_normal(98, T, (T, H), 1.0, TDT[dt])
+            flat = torch.zeros(T * H + 8, dtype=TDT[dt], device="cuda")
+            flat[off:off + T * H] = x.flatten()
+            v = flat[off:off + T * H].view(T, H)
+            assert v.is_contiguous() and v.data_ptr() % 16 == 2 * off
+            _, want = gpu.expert_run(e, x, want_f32=True)
+            y, got = gpu.expert_run(e, v, want_f32=True)
+            torch.cuda.synchronize()
+            # the same products in another fp32 order
+            assert ((got - want).norm(dim=1) / want.norm(dim=1)).max().item() < 1e-5, T
+            assert torch.equal(y, got.to(TDT[dt]))
+    finally:
+        e.free()
+
+
 def test_small_batch_expert_back_to_back(gpu, oracle):
     """Calls queued without a sync between them, alternating tokens (1..4),
     two full-size experts and a small one (other tile counts; the k-part sums

@@ -315,6 +315,35 @@ def test_plan_over_workgroups(gpu, oracle, T, K, E):
         _free(layer, experts, sh)
 
 
+@pytest.mark.parametrize("H,I,E,Ts", [(1024, 512, 256, (1, 3, 9)), (1024, 512, 64, (1, 4, 16, 40, 161)), (512, 512, 8, (700,))])
+def test_layer_rows_that_start_between_16_bytes(gpu, H, I, E, Ts):
+    """A whole layer on a view of x that starts 2 bytes past a 16-byte boundary
+    (one-token and staged decode, 64-pair items where an aligned x takes the
+    ping-pong GEMM), against its aligned copy: the same routes, the same sums."""
+    from constellation_amd.engine import Expert, Layer
+    experts = [Expert.generate(0, 210, 0x3000 + 4 * e, hidden=H, inter=I) for e in range(E)]
+    sh = Expert.generate(0, 210, 0x3000 + 4 * E, hidden=H, inter=I)
+    layer = Layer(gpu, experts, sh)
+    try:
+        w_r = gpu.gen_normal(211, 1, (E, H), 0.02, torch.bfloat16)
+        bias = gpu.gen_normal(211, 2, (E,), 0.01, torch.float32)
+        for T in Ts:
+            print(f"[moe] x at +2 bytes E={E} T={T}", flush=True)
+            x = gpu.gen_normal(212, T, (T, H), 1.0, torch.bfloat16)
+            flat = torch.zeros(T * H + 8, dtype=torch.bfloat16, device="cuda")
+            flat[1:1 + T * H] = x.flatten()
+            v = flat[1:1 + T * H].view(T, H)
+            opt = dict(n_group=8, topk_group=4, top_k=min(8, E // 2), want_f32=True)
+            _, want, ids, w = gpu.moe_layer(layer, x, w_r, bias, **opt)
+            _, got, ids2, w2 = gpu.moe_layer(layer, v, w_r, bias, **opt)
+            gpu.sync()
+            # (one token: the logits of the two pipelines are fp64 sums in another order)
+            assert torch.equal(ids, ids2) and torch.allclose(w, w2, rtol=1.2e-7, atol=0), T
+            assert ((got - want).norm(dim=1) / want.norm(dim=1)).max().item() < 1e-5, T  # another fp32 order
+    finally:
+        _free(layer, experts, sh)
+
+
 def test_many_tokens_per_resident_expert(gpu, oracle):
     """A node's share: 4 of 16 experts resident, 160 tokens x 4 routes over
     them (160 pairs per resident expert), so the LDS-ring GEMM serves the call

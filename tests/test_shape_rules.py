@@ -21,6 +21,11 @@ void expert(int t, int h, int i, int lds, size_t* out) {
 int small(int h, int i) { return expert_small_shape(h, i); }
 size_t few_bytes(int t, int i) { return few_scratch_bytes(t, i); }
 int few(int h, int i, int t, int lds) { return few_ok(h, i, t, lds); }
+int aligned(size_t p) { return dma_aligned((const void*)p); }
+void route(int t, int h, int i, int lds, int x, int gu, int dn, int* out) {
+    const ExpertRoute r = expert_route(t, h, i, lds, x, gu, dn);
+    out[0] = r.path; out[1] = r.pp_gate_up; out[2] = r.pp_down; out[3] = r.np_lds;
+}
 int few_lds(int t) { return few_gu_lds(few_tiles(t)); }
 int slices(int t, int h) { return route_slices(t, h); }
 size_t part(int t, int h, int e) { return route_part_cells(t, h, e); }
@@ -68,6 +73,31 @@ def test_few_token_kernels_fit_the_lds(rules, lds):
     """5..64 tokens where a workgroup can have the LDS, else the other kernels."""
     for T in range(1, 80):
         assert bool(rules.few(7168, 2048, T, lds)) == (5 <= T <= 64 and rules.few_lds(T) <= lds), T
+
+
+@pytest.mark.parametrize("H,I", [(7168, 2048), (1024, 512), (4096, 1536), (640, 384)])
+def test_wide_loads_only_from_aligned_rows(rules, H, I):
+    """Rows of x or weights that do not start on 16 bytes take the kernels with
+    plain loads (and the others' are not changed by them)."""
+    assert [rules.aligned(p) for p in (0, 16, 2, 4, 8, 0x7f0000000010, 0x7f000000000e)] == [1, 1, 0, 0, 0, 1, 0]
+    small, tiles, few = 1, 2, 3
+
+    def route(T, *dma):
+        out = (C.c_int * 4)()
+        rules.route(T, H, I, 160 << 10, *dma, out)
+        return tuple(out)
+
+    for T in list(range(1, 140)) + [1000]:
+        best = route(T, 1, 1, 1)
+        pp = H % 256 == 0 and T > 16 and best[0] == tiles
+        assert best[0] == (few if rules.few(H, I, T, 160 << 10) else small if T <= 4 and rules.small(H, I) else tiles)
+        assert best[1:3] == (pp, pp)
+        assert best[3] == (T if T <= (3 if H == 7168 else 4) and H % 512 == 0 else 0)
+        got = route(T, 0, 1, 1)
+        assert got == (small if best[0] == small else tiles, 0, H % 256 == 0 and T > 16, 0), T
+        if not best[0] == few:
+            assert route(T, 1, 0, 1) == best[:1] + (0,) + best[2:]
+            assert route(T, 1, 1, 0) == best[:2] + (0,) + best[3:]
 
 
 @pytest.mark.parametrize("H,E", [(7168, 256), (1024, 64), (640, 72), (384, 40), (1000, 8)])
