@@ -1122,12 +1122,6 @@ __global__ __launch_bounds__(kRouteThreads) void k_route_logits(FusedArgs A) {
 // Chunks stream through a 4-deep register ring (L2 latency is the bound).
 constexpr int kLgE = 16;       // experts per workgroup tile
 constexpr int kLgT = 32;       // tokens per workgroup tile (two MFMA column tiles)
-constexpr int kLgWaves = 8;    // K split
-constexpr int kLgRing = 4;     // chunks in flight per wave
-
-bool logits_mfma_ok(int n_tokens, int hidden) {
-    return n_tokens > kLsMaxTokens && hidden % (kLgWaves * 32 * kLgRing) == 0;
-}
 
 // 8 elements (bf16: one dwordx4; fp32: two) widened to fp64 (exact).
 template <bool F32>
@@ -1922,7 +1916,7 @@ hipError_t launch_route(const RouteArgs& R, hipStream_t s) {
     A.epl = register_epl(R.n_experts, R.n_group);
     const size_t sel = A.epl ? 0 : select_lds(R.n_experts);
     const bool xf = R.x_dtype == CX_DTYPE_F32, wf = R.w_dtype == CX_DTYPE_F32;
-    const int slices = route_slices(R.n_tokens, R.hidden);
+    const int slices = route_slices(R.n_tokens, R.hidden, R.n_experts);
     if (slices > 0) {
         const dim3 lg((R.n_experts + kLgE - 1) / kLgE, (R.n_tokens + kTileTok - 1) / kTileTok, slices);
         const dim3 blk(64 * kLsWaves);
@@ -1936,7 +1930,7 @@ hipError_t launch_route(const RouteArgs& R, hipStream_t s) {
         else if (xf) cx_launch((k_route_logits_split<true, false>), lg, blk, 0, s, A, part);
         else if (wf) cx_launch((k_route_logits_split<false, true>), lg, blk, 0, s, A, part);
         else cx_launch((k_route_logits_split<false, false>), lg, blk, 0, s, A, part);
-    } else if (logits_mfma_ok(R.n_tokens, R.hidden)) {
+    } else if (R.n_tokens > kLsMinTokens && route_mfma_ok(R.hidden)) {
         // many tokens: fp64 MFMA tiles
         const dim3 lg((R.n_experts + kLgE - 1) / kLgE, (R.n_tokens + kLgT - 1) / kLgT);
         const dim3 blk(64 * kLgWaves);

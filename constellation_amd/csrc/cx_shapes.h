@@ -125,14 +125,30 @@ inline ExpertScratch expert_scratch(int n_tokens, int hidden, int inter, int max
 }
 
 // ---------------------------------------------------------------------------
+// Router logits of many tokens in 16 x 32 tiles (k_route_logits_mfma): widths.
+constexpr int kLgWaves = 8;    // K split
+constexpr int kLgRing = 4;     // chunks in flight per wave
+
+inline bool route_mfma_ok(int hidden) { return hidden % (kLgWaves * 32 * kLgRing) == 0; }
+
 // Router logits of 4 to 256 tokens (k_route_logits_split): K slices, 0: another
-// kernel.
+// kernel.  Its 16 x 16 tiles win while one round of 256 CUs holds them: us a call
+// with them and with the 16 x 32 tiles, 256 experts 256 / 300 tokens 30.6 / 42.1 and
+// 46.9 / 42.2; 384 experts 160 / 176 / 256 tokens 137 / 150, 155 / 150 and 153 / 147;
+// 512 experts 128 / 129 / 256 tokens 34.0 / 43.8, 47.2 / 43.8 and 48.9 / 44.2.  The
+// selection reads every slice of its experts, so that above 384 experts a workgroup
+// per expert row is still the faster at 4 tokens (512 experts 18.6 against 20.8).
+// (Widths that only they and the kernel of a workgroup per expert row take keep
+// them up to 256 tokens.)
 constexpr int kLsMinTokens = 4, kLsMaxTokens = 256;
+constexpr int kLsMaxTiles = 256;
 constexpr int kLsWaves = 4;
 constexpr int kLsMaxSlices = 8;
 
-inline int route_slices(int n_tokens, int hidden) {
-    if (n_tokens < kLsMinTokens || n_tokens > kLsMaxTokens || hidden % (kLsWaves * 32) != 0) return 0;
+inline int route_slices(int n_tokens, int hidden, int n_experts) {
+    if (n_tokens < kLsMinTokens + (n_experts > 384) || n_tokens > kLsMaxTokens || hidden % (kLsWaves * 32) != 0) return 0;
+    const int tiles = (n_experts + kTileRows - 1) / kTileRows * ((n_tokens + kTileTok - 1) / kTileTok);
+    if (tiles > kLsMaxTiles && route_mfma_ok(hidden)) return 0;
     int s = n_tokens <= 32 ? 8 : n_tokens <= 64 ? 4 : n_tokens <= 128 ? 2 : 1;
     while (hidden % (kLsWaves * 32 * s) != 0) s /= 2;
     return s;

@@ -27,7 +27,7 @@ void route(int t, int h, int i, int lds, int x, int gu, int dn, int* out) {
     out[0] = r.path; out[1] = r.pp_gate_up; out[2] = r.pp_down; out[3] = r.np_lds;
 }
 int few_lds(int t) { return few_gu_lds(few_tiles(t)); }
-int slices(int t, int h) { return route_slices(t, h); }
+int slices(int t, int h, int e) { return route_slices(t, h, e); }
 size_t part(int t, int h, int e) { return route_part_cells(t, h, e); }
 size_t buffer(int t, int k, int e, int sh) { return plan_buffer_bytes(t, k, e, sh); }
 size_t plan(int t, int k, int e, int sh, int cap, int dense) {
@@ -105,8 +105,17 @@ def test_router_slices_never_shrink(rules, H, E):
     last = 0
     for T in range(1, 600):
         got = rules.part(T, H, E)
-        assert got >= last and got >= rules.slices(T, H) * T * E, T
+        assert got >= last and got >= rules.slices(T, H, E) * T * E, T
         last = got
+
+
+@pytest.mark.parametrize("H,E,least,most", [(7168, 256, 4, 256), (7168, 384, 4, 160), (1024, 512, 5, 128),
+                                            (2048, 64, 4, 256), (640, 384, 4, 256), (1000, 8, 4, 0)])
+def test_router_tiles_in_one_round(rules, H, E, least, most):
+    """The 16 x 16 tiles of the router's logits up to one round of 256 CUs, or 256
+    tokens where the 16 x 32 tiles do not take the width."""
+    for T in range(1, 300):
+        assert bool(rules.slices(T, H, E)) == (least <= T <= most), T
 
 
 @pytest.mark.parametrize("E,K", [(256, 8), (64, 8), (4, 2), (128, 1), (512, 64)])
