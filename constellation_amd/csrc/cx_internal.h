@@ -21,8 +21,6 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBigPairs = 128;  // pairs per item of the ping-pong grouped GEMM (many tokens per expert)
-constexpr int kBigMinPairs = 20;  // ... which calls of this many pairs per resident expert take
 constexpr int kWaves = 4;       // waves per workgroup
 
 // ---------------------------------------------------------------------------

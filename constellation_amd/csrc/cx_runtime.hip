@@ -669,22 +669,18 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
     const bool dec = !prefill && n_tokens <= kTileTok && dec_path_ok(layer, top_k, route);
     PlanSizes z = plan_sizes(n_tokens, top_k, layer->n_experts, layer->has_shared);
     if (dec) z.max_items = z.max_slots;  // one item per slot (<= 16 pairs each)
-    // Calls with at least kBigMinPairs pairs per resident routed expert on
-    // average take 128-pair items through the ping-pong GEMM instead of 64-pair
-    // items that each stream the expert's weights: there the matrix cores bound
-    // the work as much as HBM does.  Measured, 64-pair against 128-pair items, at
-    // 256 experts (pairs per expert: 12.5 / 16 / 20 / 24 / 28 / 32 / 47 / 128):
-    // 2119 against 2142, 2169 / 2180, 2275 / 2265, 2370 / 2338, 2469 / 2409,
-    // 2636 / 2470, 3202 / 2907 and 6997 / 5753 us a layer; at 64 experts (32 / 64
-    // / 256): 599 / 561, 915 / 738, 2655 / 2109 us.
-    // The pairs are counted on the host: exactly when the caller knows its valid
-    // routes (the wire entry point), else as every route slot, an upper bound —
-    // route tables masked to one node of several (-1 for other nodes' experts)
-    // can then take it with mostly-padding tiles (correct, slower).
+    // 128-pair items from big_min_pairs pairs per resident expert.  The pairs are
+    // counted on the host: exactly when the caller knows its valid routes (the wire
+    // entry point), else as every route slot, an upper bound.  Route tables masked to
+    // one node of several (-1 for other nodes' experts) then take them with fewer
+    // pairs (one node of four, 160 to 512 tokens: 5 to 16 pairs an expert, 494 to 528
+    // us against 494 to 543 with 64-pair items).
     const int64_t pairs = valid_routes >= 0 ? valid_routes : (int64_t)n_tokens * top_k;
     const bool x_dma = dma_aligned(x);
     const bool big = !dec && x_dma && layer->dma && pp_ok(layer->hidden, layer->inter, ctx->max_lds) &&
-                     pairs >= (int64_t)kBigMinPairs * std::max(1, layer->n_resident);
+                     pairs >= (int64_t)std::max(1, layer->n_resident) *
+                                  big_min_pairs(layer->hidden, layer->inter, layer->n_resident,
+                                                layer->has_shared != 0, ctx->n_cu > 0 ? ctx->n_cu : 256);
     if (big) {
         z.item_cap = kBigPairs;
         z.max_items = z.max_slots + (z.max_pairs + kBigPairs - 1) / kBigPairs;

@@ -85,6 +85,35 @@ inline bool pp_ok(int hidden, int inter, int max_lds) {
            inter / kKB >= kPpMinBlocks && max_lds >= kPpLds;
 }
 
+// Shapes with 64-pair grouped kernels of their own (cx_grouped.h).
+inline bool grp_shape(int hidden, int inter) {
+    const int nkg = hidden / kKB, nkd = inter / kKB;
+    return hidden % kKB == 0 && inter % kKB == 0 && (nkg == 56 || nkg == 8 || nkg == 4) && (nkd == 16 || nkd == 4);
+}
+
+// A grouped call of at least this many pairs per resident expert, on average,
+// takes 128-pair items through the ping-pong GEMM: there the matrix cores bound
+// the work as much as HBM does, and 64-pair items stream an expert's weights once
+// for each.  us a layer with 64 and with 128-pair items at 20 / 32 / 48 / 64 / 80 /
+// 128 pairs per expert, 7168 x 2048 with the shared expert:
+//   256 experts  2226 2524 3037 3917 4909 6704   2153 2354 2630 3154 3559 5357
+//   64 experts   614 666 783 982 1243 1660       624 713 778 864 937 1406
+//   64, none shared  535 598 708 904 1132 1514   523 569 622 741 816 1276
+// The shared expert's items, all full, run last: where the others last for few
+// rounds of the CUs, 128 pairs at the end cost more than fewer reads of the weights
+// save, up to 79 pairs (8 experts, which fit one round, gain from 20: 121 / 105).
+// Rows of few blocks gain as late, a ring's fill and drain being a larger part of an
+// item: 512 x 7168 (inter x hidden), 256 experts 683 765 908 1171 1488 and 732 807
+// 936 1048 1181; and below two rounds the halved count of workgroups shows too (1024
+// x 512, 16 experts, 96 pairs 45 against 52), up to the 128 pairs of a full item.
+constexpr int kBigPairs = 128;
+inline int big_min_pairs(int hidden, int inter, int n_resident, bool shared, int n_cu) {
+    if (!grp_shape(hidden, inter)) return 20;
+    const int wgs = (n_resident + (shared ? 1 : 0)) * (inter / kPpRowsGu);  // gate/up, an item each
+    if (hidden / kKB == 56 && inter / kKB == 16) return !shared || wgs <= n_cu || wgs >= 8 * n_cu ? 20 : 80;
+    return wgs >= 2 * n_cu ? 80 : kBigPairs;
+}
+
 // Kernels of one expert on the fast paths.  Above 16 tokens the 64-token items of
 // the grouped kernels leave most CUs idle (16 gate/up workgroups at 17..64
 // tokens): 66 / 108 us at 32 / 300 tokens against 42 / 59 with the ping-pong GEMM.

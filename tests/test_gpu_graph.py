@@ -78,7 +78,7 @@ def test_moe_layer_graph_replays_equal_eager(gpu, T):
 def _smaller_calls(gpu, kind, H, I, E):
     """(tokens of the largest call, smaller ones, call(T, context) -> outputs, cleanup)."""
     from constellation_amd.engine import Expert, Layer
-    x = gpu.gen_normal(131, 1, (700, H), 1.0, torch.bfloat16)
+    x = gpu.gen_normal(131, 1, (1100, H), 1.0, torch.bfloat16)
     w_r = gpu.gen_normal(131, 2, (E, H), 0.02, torch.bfloat16)
     bias = gpu.gen_normal(131, 3, (E,), 0.01, torch.float32)
     opt = dict(n_group=8, topk_group=4, top_k=8)
@@ -98,7 +98,7 @@ def _smaller_calls(gpu, kind, H, I, E):
     def call(T, c):
         y, _, ids, w = c.moe_layer(layer, x[:T], w_r, bias, **opt)
         return y, ids, w
-    return 161, (160, 159, 100, 40, 17, 16, 8, 1), call, free
+    return 1100, (1024, 1023, 300, 40, 17, 16, 8, 1), call, free  # 128-pair items from 1024
 
 
 @pytest.mark.parametrize("kind", ["route", "expert", "layer"])

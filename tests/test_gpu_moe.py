@@ -221,13 +221,19 @@ def test_moe_many_tokens_per_expert(gpu, oracle, H, I, E, T, K, dtype, shared):
     (1024, 1024, (33, 64, 65, 16), torch.float16),
     (1024, 512, (48, 80, 81, 129), torch.bfloat16),
     (512, 2048, (96, 97, 112, 32), torch.bfloat16),
-    (2048, 512, (113, 127, 256, 2), torch.float16)])
+    (2048, 512, (113, 127, 256, 2), torch.float16),
+    (512, 640, (1, 17, 128), torch.bfloat16),          # as above, at shapes with no 64-pair kernels
+    (768, 640, (48, 80, 81, 129), torch.bfloat16),     # (odd counts of blocks among them)
+    (1280, 1920, (96, 97, 112, 32), torch.float16),
+    (768, 1408, (33, 64, 65, 16), torch.bfloat16)])
 def test_item_sizes_of_the_ping_pong_gemm(gpu, oracle, H, I, counts, dtype):
     """Experts of exactly `counts` tokens each: every column-tile count of an
-    item and its edges, one and two items per expert, against the oracle."""
+    item and its edges, one and two items per expert, against the oracle.  The
+    shapes with 64-pair kernels of their own (hidden 512 and 1024, inter 512 and
+    2048) take those at these counts, the others the ping-pong GEMM."""
     print(f"[moe] item sizes H={H} I={I} counts={counts}", flush=True)
     E, T = len(counts), sum(counts)
-    assert T >= 32 * E  # the rule for 128-pair items
+    assert T >= 20 * E  # 128-pair items, where there are no 64-pair kernels
     layer, experts, sh, cpu, cpu_sh = _make_layer(gpu, oracle, E, H, I, seed=150 + E, shared=False)
     try:
         x = gpu.gen_normal(151 + T, 1, (T, H), 1.0, dtype)
@@ -247,15 +253,17 @@ def test_item_sizes_of_the_ping_pong_gemm(gpu, oracle, H, I, counts, dtype):
         _free(layer, experts, sh)
 
 
-@pytest.mark.parametrize("n,T", [(62, 156), (63, 159), (64, 160), (149, 373)])
-def test_ping_pong_tiles_over_the_xcds(gpu, oracle, n, T):
+@pytest.mark.parametrize("n,T,I", [(62, 156, 512), (63, 159, 512), (64, 160, 512), (149, 373, 512),
+                                   (40, 100, 640), (62, 156, 640), (63, 159, 640), (126, 315, 640), (149, 373, 640)])
+def test_ping_pong_tiles_over_the_xcds(gpu, oracle, n, T, I):
     """n experts and the shared one, one 128-pair item each but for the shared
-    one's, four row tiles an item: fewer than 256 workgroups, 256 and a little
-    more, and 512 with a rest, so that every branch of the tile -> XCD mapping
-    is met; against the oracle."""
+    one's, five (gate/up) and four (down) row tiles an item at inter 640: fewer
+    than 256 workgroups, 256 and a little more, 512 and a rest, so that every
+    branch of the tile -> XCD mapping is met; against the oracle.  (Inter 512 has
+    64-pair kernels of its own, which it takes at these counts.)"""
     print(f"[moe] tiles over the XCDs n={n}", flush=True)
-    H, I, K = 1024, 512, 8
-    assert 20 * n <= T * K < 128 * n  # the rule for 128-pair items, one item an expert
+    H, K = 1024, 8
+    assert 20 * n <= T * K < 128 * n  # 128-pair items (inter 640), one item an expert
     layer, experts, sh, cpu, cpu_sh = _make_layer(gpu, oracle, n, H, I, seed=180 + n, shared=True)
     try:
         x = gpu.gen_normal(181, n, (T, H), 1.0, torch.bfloat16)
@@ -280,7 +288,7 @@ def test_plan_over_workgroups(gpu, oracle, T, K, E):
     share only: dropped, and reported by the sync."""
     print(f"[moe] plan T={T} K={K} E={E}", flush=True)
     from constellation_amd._lib import CxError
-    H, I = 512, 512
+    H, I = 512, 640  # no 64-pair kernels: 128-pair items from 20 pairs per expert
     layer, experts, sh, cpu, cpu_sh = _make_layer(gpu, oracle, E, H, I, seed=190 + E, shared=True)
     try:
         x = gpu.gen_normal(191, T, (T, H), 1.0, torch.bfloat16)

@@ -26,6 +26,7 @@ void route(int t, int h, int i, int lds, int x, int gu, int dn, int* out) {
     const ExpertRoute r = expert_route(t, h, i, lds, x, gu, dn);
     out[0] = r.path; out[1] = r.pp_gate_up; out[2] = r.pp_down; out[3] = r.np_lds;
 }
+int big(int h, int i, int n, int sh) { return big_min_pairs(h, i, n, sh, 256); }
 int few_lds(int t) { return few_gu_lds(few_tiles(t)); }
 int slices(int t, int h, int e) { return route_slices(t, h, e); }
 size_t part(int t, int h, int e) { return route_part_cells(t, h, e); }
@@ -107,6 +108,16 @@ def test_router_slices_never_shrink(rules, H, E):
         got = rules.part(T, H, E)
         assert got >= last and got >= rules.slices(T, H, E) * T * E, T
         last = got
+
+
+@pytest.mark.parametrize("H,I,n,shared,pairs", [
+    (7168, 2048, 256, 1, 20), (7168, 2048, 127, 1, 20), (7168, 2048, 64, 0, 20), (7168, 2048, 4, 0, 20),
+    (7168, 2048, 64, 1, 80), (7168, 2048, 16, 1, 80), (7168, 2048, 15, 1, 20),  # the shared expert's items last
+    (7168, 512, 256, 1, 80), (1024, 2048, 64, 0, 80), (1024, 512, 64, 1, 128), (512, 512, 8, 0, 128),  # few blocks
+    (2048, 768, 128, 1, 20), (4096, 1536, 8, 1, 20), (2048, 512, 64, 1, 20)])  # no 64-pair kernels
+def test_pairs_per_expert_of_128_pair_items(rules, H, I, n, shared, pairs):
+    """The least pairs per resident expert for 128-pair items, on 256 CUs."""
+    assert rules.big(H, I, n, shared) == pairs
 
 
 @pytest.mark.parametrize("H,E,least,most", [(7168, 256, 4, 256), (7168, 384, 4, 160), (1024, 512, 5, 128),
