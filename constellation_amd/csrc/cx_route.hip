@@ -702,11 +702,15 @@ __device__ __forceinline__ int plan_first_item(int n, int item_cap) {
 // every G-th slot and its part of the shared expert's.  What bounds one
 // workgroup is its scattered 4-byte stores (three per route) and their LDS
 // cursors; the count that all repeat reads the routes from L2 in 16-byte loads.
-// us a plan, in one workgroup with the routes staged in LDS and
-// now, 8 routes a token: 17 / 64 / 256 / 1024 / 2048 tokens of one node of four
-// 9.0 -> 7.9, 10.9 -> 7.9, 12.3 -> 9.2, 29 -> 11.5, 52 -> 13.8.
+// Up to 1024 routes, one workgroup, each thread keeps its one route in registers
+// from the count to the stores; reading the routes again there and comparing them
+// for repeats in memory cost 1 to 3 us of chained loads (64 experts, 17 / 32 / 128
+// tokens of 8 routes: 9.2 / 8.8 / 8.2 us so, 5.9 / 6.0 / 7.0 now).
+// us a plan of 8 routes a token, 256 experts, in one workgroup with the routes
+// staged in LDS and now: 17 / 64 / 128 / 256 / 1024 / 2048 tokens 7.5 -> 6.4, 9.3 ->
+// 7.1, 8.6 -> 8.1, 12.0 -> 9.2, 31 -> 9.9, 63 -> 11.6.
 // LDS: first pair, cursor and first item of every expert (3 E ints).
-constexpr int kPlanShare = 1024;  // routes per workgroup
+constexpr int kPlanShare = kPlanThreads;  // routes per workgroup
 constexpr int kPlanMaxWgs = 64;
 
 struct Scan3 {
@@ -756,18 +760,25 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(const int32_t* __restrict
                                                             int* err_flag) {
     extern __shared__ int plan_lds[];
     __shared__ int tmp[3 * 33];
+    __shared__ int one_id[kPlanThreads];
     const int E = n_experts, T = n_tokens, K = top_k, tid = threadIdx.x, nt = blockDim.x;
     const int G = gridDim.x, b = blockIdx.x;
     int* cur = plan_lds;    // routes before this share; later the next pair of the share
     int* first = cur + E;   // routes from this share on; later the expert's first pair
     int* item = first + E;  // residency; later 2 x first item + (its first item is a half one)
     const int share = (T + G - 1) / G, t0 = min(b * share, T), t1 = min(t0 + share, T);
+    // up to a route per thread (one workgroup): read once, beside the residency
+    const bool one = T * K <= nt, own = one && tid < T * K;
+    const int own_id = own ? ids[tid] : -1;
+    const float own_w = own ? w[tid] : 0.f;
+    bool own_ok = false;
     for (int e = tid; e < E; e += nt) {
         cur[e] = first[e] = 0;
         item[e] = table[e].w_up != nullptr ? 1 : 0;
     }
     const bool shared = has_shared && table[E].w_up != nullptr;
     const int s0 = shared ? T : 0;  // first routed pair
+    if (one) one_id[tid] = own_id;
     __syncthreads();
     // 1) counts of valid routes
     int err = 0;
@@ -778,7 +789,12 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(const int32_t* __restrict
         err |= bad;
         return bad == 0;
     };
-    if (K == 8) {
+    if (one) {
+        bool dup = false;
+        for (int j = own ? tid / K * K : tid; j < tid; ++j) dup |= one_id[j] == own_id;
+        own_ok = check(own_id, own_w, dup);
+        if (own_ok) atomicAdd(&first[own_id], 1);
+    } else if (K == 8) {
         for (int t = tid; t < T; t += nt) {
             Route4 r[2], x[2];
 #pragma unroll
@@ -882,16 +898,25 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(const int32_t* __restrict
         const int j = rank < f ? rank : (rank - f) % item_cap;
         if (j < 4 && first_item + i < max_items) P.item_rec[first_item + i].tok[j] = t;
     };
-    for (int j = tid; j < (t1 - t0) * K; j += nt) {
-        const int i = t0 * K + j, e = ids[i], t = i / K;
+    auto put_route = [&](int i, int e, float wt, bool ok) {
+        const int t = i / K;
         int pos = -1;
-        if (e >= 0 && e < E && item[e] >= 0 && !dup_route(ids, i, K) && route_weight_ok(w[i])) {
+        if (ok) {
             pos = atomicAdd(&cur[e], 1);
             P.pair_token[pos] = t;
-            P.pair_weight[pos] = w[i];
+            P.pair_weight[pos] = wt;
             put_token(item[e] >> 1, item[e] & 1, pos - first[e], t);
         }
         P.token_pairs[(size_t)t * (K + 1) + (i - t * K)] = pos;
+    };
+    if (one) {
+        if (own) put_route(tid, own_id, own_w, own_ok);
+    } else {
+        for (int i = t0 * K + tid; i < t1 * K; i += nt) {
+            const int e = ids[i];
+            const float wt = w[i];
+            put_route(i, e, wt, e >= 0 && e < E && item[e] >= 0 && !dup_route(ids, i, K) && route_weight_ok(wt));
+        }
     }
     for (int t = t0 + tid; t < t1; t += nt) {
         if (shared) {
@@ -1960,7 +1985,9 @@ hipError_t launch_plan(const int32_t* ids, const float* w, int n_tokens, int top
                        int max_items, PlanPtrs plan, int* err_flag, hipStream_t s) {
     const int wgs = std::max(1, std::min(kPlanMaxWgs, (n_tokens * top_k + kPlanShare - 1) / kPlanShare));
     const size_t lds = sizeof(int) * 3 * (size_t)n_experts;
-    cx_launch(k_plan, dim3(wgs), dim3(kPlanThreads), lds, s, ids, w, n_tokens, top_k, table,
+    // (256 threads: barriers of 4 waves instead of 16; 8 experts, 64 routes 5.5 -> 5.1 us)
+    const int threads = n_tokens * top_k <= 256 && n_experts <= 256 ? 256 : kPlanThreads;
+    cx_launch(k_plan, dim3(wgs), dim3(threads), lds, s, ids, w, n_tokens, top_k, table,
               n_experts, has_shared, item_cap, max_items, plan, err_flag);
     return hipGetLastError();
 }

@@ -279,9 +279,11 @@ def test_ping_pong_tiles_over_the_xcds(gpu, oracle, n, T, I):
         _free(layer, experts, sh)
 
 
-@pytest.mark.parametrize("T,K,E", [(127, 8, 16), (128, 8, 16), (129, 8, 16), (257, 8, 24), (300, 5, 16), (1025, 1, 3)])
+@pytest.mark.parametrize("T,K,E", [(127, 8, 16), (128, 8, 16), (129, 8, 16), (257, 8, 24), (300, 5, 16), (1025, 1, 3),
+                                   (32, 8, 16), (33, 8, 16), (51, 5, 16), (1024, 1, 3)])
 def test_plan_over_workgroups(gpu, oracle, T, K, E):
-    """Plans of one to three workgroups around the 1024 routes that each takes,
+    """Plans of one to three workgroups around the 1024 routes that each takes (a
+    route per thread in one of them, of 256 threads up to 256 routes),
     8 routes a token (16-byte loads, here from a 4-byte aligned view) and other
     counts, absent routes, experts of 129 to 1025 tokens whose first 128-pair
     item is halved; every token against the oracle.  Then faults in the last
