@@ -240,6 +240,8 @@ struct RouteArgs {
     float scale;
     double* logits;         // scratch [T, E]
     double* part;           // scratch [route_slices, T, E] (launch_route, where that is above 1)
+    double* scores;         // scratch [2, E] (one-token decode)
+    float* gu_part;         // scratch: the shared expert's k-part sums (decode)
     int32_t* ids;           // [T, top_k]
     float* wout;            // [T, top_k]
     // planner (nullable plan = route only)

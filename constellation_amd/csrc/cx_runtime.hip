@@ -231,9 +231,9 @@ struct cx_ctx {
     int* err_flag = nullptr;           // device int: error bits of the device checks
     int max_lds = 65536;               // dynamic LDS budget per workgroup
     int n_cu = 0;                      // compute units (0: unknown)
-    DevBuf plan_buf, hhi, hlo, ypart, logits, route_part, route_ids, route_w, hscratch;
-    DevBuf gu_part;                    // k-part gate/up sums (1..4 tokens of an expert; decode's shared expert)
-    DevBuf scores;                     // one-token router scores s, c [E][2] fp64 (decode)
+    DevBuf plan_buf, hhi, hlo, ypart, route_ids, route_w;
+    DevBuf one;                        // scratch of one expert (expert_scratch_bytes)
+    DevBuf logits;                     // router scratch (RouteScratch), the logits first
     int route_T = 0, route_E = 0;      // shape of the fp64 logits of the last router call
     DevBuf dx, dy;                     // cx_expert_run_host staging (device)
     void* pin_x = nullptr;             // pinned host staging
@@ -366,19 +366,15 @@ int check_desc(const cx_expert_desc* e) {
 struct ExpertPlan {
     ExpertLaunch L;
     ExpertRoute route;
-    size_t h_f32_bytes;   // generic path: fp32 h [T, I]
-    size_t h_plane_bytes; // tile paths: each bf16 plane h_hi / h_lo [T, I]
-    size_t h_frag_bytes;  // few-token path: h in fragment order
-    size_t gu_part_bytes; // small path: k-part gate/up sums [2][2][T][I] fp32
+    size_t scratch_bytes;  // what the path needs
 };
 
 ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int n_tokens,
                        void* y, int out_dtype, float* y_f32, int max_lds, int n_cu) {
     ExpertPlan P{};
-    const size_t TI = (size_t)n_tokens * e.inter;
     if (!fast_path_ok(e)) {
         P.route.path = kPathGeneric;
-        P.h_f32_bytes = TI * 4;
+        P.scratch_bytes = expert_call_bytes(kPathGeneric, n_tokens, e.inter);
         return P;
     }
     ExpertLaunch& L = P.L;
@@ -398,30 +394,22 @@ ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int
     P.route = expert_route(n_tokens, e.hidden, e.inter, max_lds, dma_aligned(x),
                            dma_aligned(e.w_gate) && dma_aligned(e.w_up), dma_aligned(e.w_down));
     L.np_lds = P.route.np_lds;
-    if (P.route.path == kPathFew) {
-        P.h_frag_bytes = few_scratch_bytes(n_tokens, e.inter);
-    } else if (P.route.path == kPathSmall) {
-        P.gu_part_bytes = sizeof(float) * 2 * 2 * TI;
-        L.gu_kparts = 2;
-    } else {
-        P.h_plane_bytes = TI * 2;
-    }
+    if (P.route.path == kPathSmall) L.gu_kparts = 2;
+    P.scratch_bytes = expert_call_bytes(P.route.path, n_tokens, e.inter);
     return P;
 }
 
-// Launches a planned expert on `s`; the scratch pointers the path needs are
-// set (h_f32 / h_hi + h_lo / h_hi for h in fragment order / gu_part).  ctx
-// (nullable) only collects timing.
+// Launches a planned expert on `s` with P.scratch_bytes of scratch (256-byte
+// aligned).  ctx (nullable) only collects timing.
 int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* x, int in_dtype,
-               int n_tokens, void* y, int out_dtype, float* y_f32, float* h_f32, uint16_t* h_hi,
-               uint16_t* h_lo, float* gu_part, hipStream_t s) {
+               int n_tokens, void* y, int out_dtype, float* y_f32, void* scratch, hipStream_t s) {
     if (P.route.path == kPathGeneric) {
-        CX_HIP(launch_generic_expert(e, x, in_dtype, n_tokens, h_f32, y, out_dtype, y_f32, s));
+        CX_HIP(launch_generic_expert(e, x, in_dtype, n_tokens, static_cast<float*>(scratch), y, out_dtype, y_f32, s));
         return CX_OK;
     }
     ExpertLaunch& L = P.L;
     if (P.route.path == kPathSmall) {
-        L.gu_part = gu_part;
+        L.gu_part = static_cast<float*>(scratch);
         {
             Span sp(ctx, "gate_up", s);
             CX_HIP(launch_gate_up_kpart(L, s));
@@ -430,8 +418,8 @@ int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* 
         CX_HIP(launch_down_ks(L, s));
         return CX_OK;
     }
-    L.h_hi = h_hi;
-    L.h_lo = h_lo;
+    L.h_hi = static_cast<uint16_t*>(scratch);
+    L.h_lo = reinterpret_cast<uint16_t*>(static_cast<char*>(scratch) + h_lo_offset(n_tokens, e.inter));  // (not few)
     if (P.route.path == kPathFew) {
         {
             Span sp(ctx, "gate_up", s);
@@ -546,7 +534,7 @@ int moe_decode(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, 
     const bool split = route != nullptr && sg != nullptr &&
                        dec_shared_split_ok(layer->hidden, layer->inter, T);
     if (split) {
-        SG.gu_part = static_cast<float*>(ctx->gu_part.p);
+        SG.gu_part = route->gu_part;
         SG.gu_kparts = 2;
     }
     const int routed_items = std::min(T * top_k, layer->n_experts);
@@ -562,7 +550,7 @@ int moe_decode(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, 
                        down_comb1_ok(layer->hidden, layer->inter, top_k, ctx->max_lds) &&
                        dec_fused_sel_ok(route->n_experts, route->n_group, route->topk_group,
                                         layer->hidden, top_k, route->x_dtype);
-    double* sc = fused ? static_cast<double*>(ctx->scores.p) : nullptr;
+    double* sc = fused ? route->scores : nullptr;
     if (route != nullptr) {
         route->plan = &P;
         route->table = layer->table;
@@ -639,13 +627,19 @@ int moe_decode(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, 
     return CX_OK;
 }
 
-// Scratch of launch_route beside the logits.
-int route_part(cx_ctx* ctx, RouteArgs* R, hipStream_t s) {
-    const size_t cells = route_part_cells(R->n_tokens, R->hidden, R->n_experts);
-    if (cells == 0) return CX_OK;
-    const int rc = ensure(&ctx->route_part, cells * sizeof(double), s);
-    R->part = static_cast<double*>(ctx->route_part.p);
-    return rc;
+// Scratch of a router call (RouteScratch).
+int reserve_route(cx_ctx* ctx, RouteArgs* R, bool decode, int dec_inter, hipStream_t s) {
+    const RouteScratch z = route_scratch(R->n_tokens, R->hidden, R->n_experts, decode, dec_inter);
+    const int rc = ensure(&ctx->logits, z.bytes, s);
+    if (rc) return rc;
+    char* p = static_cast<char*>(ctx->logits.p);
+    R->logits = reinterpret_cast<double*>(p);
+    R->part = reinterpret_cast<double*>(p + z.part);
+    R->scores = reinterpret_cast<double*>(p + z.scores);
+    R->gu_part = reinterpret_cast<float*>(p + z.gu_part);
+    ctx->route_T = R->n_tokens;
+    ctx->route_E = R->n_experts;
+    return CX_OK;
 }
 
 // Routed-expert compute; when `route` is given, the router runs first on the
@@ -692,11 +686,9 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
     if ((rc = ensure(&ctx->hhi, (size_t)z.max_pairs * I * 2, s))) return rc;
     if ((rc = ensure(&ctx->hlo, (size_t)z.max_pairs * I * 2, s))) return rc;
     if ((rc = ensure(&ctx->ypart, (size_t)z.max_pairs * H * 4, s))) return rc;
-    if (route != nullptr && dec_path_ok(layer, top_k, route)) {  // what moe_decode needs with the router
-        const size_t t = std::min(n_tokens, kDecSplitMaxTokens);
-        if ((layer->has_shared && (rc = ensure(&ctx->gu_part, sizeof(float) * 2 * 2 * t * I, s))) ||
-            (rc = ensure(&ctx->scores, sizeof(double) * 2 * (size_t)layer->n_experts, s)))
-            return rc;
+    if (route != nullptr) {
+        const bool decode = dec_path_ok(layer, top_k, route);
+        if ((rc = reserve_route(ctx, route, decode, layer->has_shared ? layer->inter : 0, s))) return rc;
     }
     if (dec)
         return moe_decode(ctx, layer, x, in_dtype, n_tokens, ids, w, top_k, y, out_dtype, y_f32,
@@ -708,7 +700,6 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
         route->item_cap = z.item_cap;
         route->max_items = z.max_items;
         route->err_flag = ctx->err_flag;
-        if ((rc = route_part(ctx, route, s))) return rc;
         Span sp(ctx, "route", s);
         CX_HIP(launch_route(*route, s));
     } else {
@@ -752,7 +743,7 @@ int moe_run(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype, int
 int fill_route(cx_ctx* ctx, const void* x, int x_dtype, const void* w_router, int w_dtype,
                const float* bias, const uint8_t* resident, int n_tokens, int hidden,
                int n_experts, int n_group, int topk_group, int top_k, int norm,
-               float scale, int32_t* ids, float* wout, hipStream_t s, RouteArgs* R) {
+               float scale, int32_t* ids, float* wout, RouteArgs* R) {
     if (!ctx) return fail(CX_EINVAL, "NULL context");
     if (!x || !w_router || !bias || !ids || !wout) return fail(CX_EINVAL, "NULL buffer");
     if ((x_dtype != CX_DTYPE_BF16 && x_dtype != CX_DTYPE_F32) ||
@@ -769,9 +760,6 @@ int fill_route(cx_ctx* ctx, const void* x, int x_dtype, const void* w_router, in
         return fail(CX_EINVAL, "invalid top_k=%d for num_experts=%d", top_k, n_experts);
     int rc = set_device(ctx->device);
     if (rc) return rc;
-    if ((rc = ensure(&ctx->logits, (size_t)n_tokens * n_experts * 8, s))) return rc;
-    ctx->route_T = n_tokens;
-    ctx->route_E = n_experts;
     *R = RouteArgs{};
     R->x = x;
     R->x_dtype = x_dtype;
@@ -787,7 +775,6 @@ int fill_route(cx_ctx* ctx, const void* x, int x_dtype, const void* w_router, in
     R->top_k = top_k;
     R->norm = norm;
     R->scale = scale;
-    R->logits = static_cast<double*>(ctx->logits.p);
     R->ids = ids;
     R->wout = wout;
     return CX_OK;
@@ -1067,8 +1054,8 @@ int cx_ctx_destroy(cx_ctx* c) {
     (void)hipSetDevice(c->device);
     (void)hipDeviceSynchronize();
     drain_spans(c);
-    DevBuf* bufs[] = {&c->plan_buf, &c->hhi, &c->hlo, &c->ypart, &c->logits, &c->route_part, &c->route_ids,
-                      &c->route_w, &c->hscratch, &c->gu_part, &c->scores, &c->dx, &c->dy};
+    DevBuf* bufs[] = {&c->plan_buf, &c->hhi, &c->hlo, &c->ypart, &c->one, &c->logits, &c->route_ids,
+                      &c->route_w, &c->dx, &c->dy};
     for (DevBuf* b : bufs)
         if (b->p) (void)hipFree(b->p);
     if (c->err_flag) (void)hipFree(c->err_flag);
@@ -1131,16 +1118,11 @@ int cx_expert_run(cx_ctx* ctx, const cx_expert_desc* expert, const void* x, int 
     if ((rc = set_device(ctx->device))) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->max_lds, ctx->n_cu);
-    if (P.h_f32_bytes && (rc = ensure(&ctx->hscratch, P.h_f32_bytes, s))) return rc;
-    if (P.route.path != kPathGeneric) {
-        const ExpertScratch z = expert_scratch(n_tokens, expert->hidden, expert->inter, ctx->max_lds);
-        if ((z.h_hi && (rc = ensure(&ctx->hhi, z.h_hi, s))) || (z.h_lo && (rc = ensure(&ctx->hlo, z.h_lo, s))) ||
-            (z.gu_part && (rc = ensure(&ctx->gu_part, z.gu_part, s))))
-            return rc;
-    }
-    return run_expert(ctx, P, *expert, x, in_dtype, n_tokens, y, out_dtype, y_f32,
-                      static_cast<float*>(ctx->hscratch.p), static_cast<uint16_t*>(ctx->hhi.p),
-                      static_cast<uint16_t*>(ctx->hlo.p), static_cast<float*>(ctx->gu_part.p), s);
+    const size_t bytes = P.route.path == kPathGeneric
+                             ? P.scratch_bytes
+                             : expert_scratch_bytes(n_tokens, expert->hidden, expert->inter, ctx->max_lds);
+    if ((rc = ensure(&ctx->one, bytes, s))) return rc;
+    return run_expert(ctx, P, *expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->one.p, s);
 }
 
 int cx_expert_run_static(int device, const cx_expert_desc* expert, const void* x, int in_dtype,
@@ -1155,18 +1137,13 @@ int cx_expert_run_static(int device, const cx_expert_desc* expert, const void* x
     int max_lds = 0, n_cu = 0;
     if ((rc = static_scratch(device, &base, &max_lds, &n_cu))) return rc;
     ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, max_lds, n_cu);
-    // one region per path: fp32 h, or h_hi then h_lo (256-B aligned), or h in
-    // fragment order, or the part sums
-    const size_t lo_off = (P.h_plane_bytes + 255) & ~(size_t)255;
-    const size_t need = std::max({P.h_f32_bytes, lo_off + P.h_plane_bytes, P.h_frag_bytes, P.gu_part_bytes});
+    const size_t need = P.scratch_bytes;
     if (need > CX_STATIC_SCRATCH_BYTES)
         return fail(CX_EINVAL,
                     "cx_expert_run_static: %d tokens x inter %d need %zu scratch bytes, "
                     "more than the static %d (use cx_expert_run)",
                     n_tokens, expert->inter, need, (int)CX_STATIC_SCRATCH_BYTES);
-    return run_expert(nullptr, P, *expert, x, in_dtype, n_tokens, y, out_dtype, y_f32,
-                      reinterpret_cast<float*>(base), reinterpret_cast<uint16_t*>(base),
-                      reinterpret_cast<uint16_t*>(base + lo_off), reinterpret_cast<float*>(base),
+    return run_expert(nullptr, P, *expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, base,
                       static_cast<hipStream_t>(stream));
 }
 
@@ -1280,8 +1257,8 @@ int cx_route(cx_ctx* ctx, const void* x, int x_dtype, const void* w_router, int 
     RouteArgs R{};
     int rc = fill_route(ctx, x, x_dtype, w_router, w_dtype, bias, resident, n_tokens, hidden,
                         n_experts, n_group, topk_group, top_k, norm_topk_prob,
-                        routed_scaling_factor, topk_ids, topk_w, s, &R);
-    if (rc || (rc = route_part(ctx, &R, s))) return rc;
+                        routed_scaling_factor, topk_ids, topk_w, &R);
+    if (rc || (rc = reserve_route(ctx, &R, false, 0, s))) return rc;
     Span sp(ctx, "route", s);
     CX_HIP(launch_route(R, s));
     return CX_OK;
@@ -1337,7 +1314,7 @@ int cx_moe_layer(cx_ctx* ctx, const cx_layer* layer, const void* x, int in_dtype
     RouteArgs R{};
     if ((rc = fill_route(ctx, x, in_dtype, w_router, w_dtype, bias, resident, n_tokens,
                          layer->hidden, layer->n_experts, n_group, topk_group, top_k,
-                         norm_topk_prob, routed_scaling_factor, ids, w, s, &R)))
+                         norm_topk_prob, routed_scaling_factor, ids, w, &R)))
         return rc;
     return moe_run(ctx, layer, x, in_dtype, n_tokens, ids, w, top_k, y, out_dtype, y_f32, s,
                    n_tokens > kTileTok, &R);

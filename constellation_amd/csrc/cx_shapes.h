@@ -6,6 +6,8 @@
 // captured graph may still use.  So what a call asks for covers every call of
 // the same entry point and shape with fewer tokens, whatever kernels these take:
 // a program that has run its largest call allocates no more, under capture too.
+// Parts that belong together share one allocation: a context's first call pays
+// for each.
 #pragma once
 
 #include <algorithm>
@@ -139,18 +141,29 @@ inline ExpertRoute expert_route(int n_tokens, int hidden, int inter, int max_lds
     return r;
 }
 
-// Context scratch of a call of cx_expert_run on the fast paths: h as two bf16
-// planes, or all of it in h_hi in fragment order; fp32 k-part sums.
-struct ExpertScratch {
-    size_t h_hi, h_lo, gu_part;
-};
+// Scratch of a call on one expert: h in fp32 (generic kernels), in fragment order
+// (few-token path), as fp32 k-part sums of gate and up (1..4 tokens), or as two
+// bf16 planes, the lo plane at h_lo_offset.
+constexpr size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+constexpr size_t gu_part_bytes(int n_tokens, int inter) { return sizeof(float) * 2 * 2 * (size_t)n_tokens * inter; }
+constexpr size_t h_lo_offset(int n_tokens, int inter) { return align256((size_t)n_tokens * inter * 2); }
 
-inline ExpertScratch expert_scratch(int n_tokens, int hidden, int inter, int max_lds) {
+inline size_t expert_call_bytes(ExpertPath path, int n_tokens, int inter) {
+    switch (path) {
+        case kPathGeneric: return (size_t)n_tokens * inter * 4;
+        case kPathSmall: return gu_part_bytes(n_tokens, inter);
+        case kPathFew: return few_scratch_bytes(n_tokens, inter);
+        default: return h_lo_offset(n_tokens, inter) + (size_t)n_tokens * inter * 2;
+    }
+}
+
+// The same of a context, for the paths of all calls with up to n_tokens tokens.
+inline size_t expert_scratch_bytes(int n_tokens, int hidden, int inter, int max_lds) {
     const bool small = expert_small_shape(hidden, inter);
-    const size_t plane = small && n_tokens <= kDownKsRows ? 0 : (size_t)n_tokens * inter * 2;
     const int few = std::min(n_tokens, few_max_tokens(max_lds));
-    return {std::max(plane, few_ok(hidden, inter, few, max_lds) ? few_scratch_bytes(few, inter) : 0), plane,
-            small ? sizeof(float) * 2 * 2 * (size_t)std::min(n_tokens, kDownKsRows) * inter : 0};
+    return std::max({small ? expert_call_bytes(kPathSmall, std::min(n_tokens, kDownKsRows), inter) : 0,
+                     few_ok(hidden, inter, few, max_lds) ? expert_call_bytes(kPathFew, few, inter) : 0,
+                     small && n_tokens <= kDownKsRows ? 0 : expert_call_bytes(kPathTiles, n_tokens, inter)});
 }
 
 // ---------------------------------------------------------------------------
@@ -183,11 +196,25 @@ inline int route_slices(int n_tokens, int hidden, int n_experts) {
     return s;
 }
 
-// fp64 cells of the slices: slices x tokens is at most 256 (8 x 32, 4 x 64, 2 x 128).
+// Scratch of a router call, offsets in bytes: logits [T, E] in fp64; their slices
+// (slices x tokens is at most 256: 8 x 32, 4 x 64, 2 x 128); and for a layer with a
+// decode pipeline (`decode`) its one-token scores s, c [E] and, with a shared
+// expert, the k-part gate/up sums of up to kDecSplitMaxTokens tokens (dec_inter: its
+// inter, else 0).  Up to 16 tokens of such a layer need no slices.
 constexpr int kLsPartTokens = 256;
 
-inline size_t route_part_cells(int n_tokens, int hidden, int n_experts) {
-    return n_tokens >= kLsMinTokens && hidden % (kLsWaves * 32) == 0 ? (size_t)kLsPartTokens * n_experts : 0;
+struct RouteScratch {
+    size_t part, scores, gu_part, bytes;
+};
+
+inline RouteScratch route_scratch(int n_tokens, int hidden, int n_experts, bool decode, int dec_inter) {
+    const bool part = n_tokens >= kLsMinTokens && hidden % (kLsWaves * 32) == 0 && !(decode && n_tokens <= kTileTok);
+    RouteScratch z;
+    z.part = align256(sizeof(double) * (size_t)n_tokens * n_experts);
+    z.scores = z.part + align256(part ? sizeof(double) * kLsPartTokens * (size_t)n_experts : 0);
+    z.gu_part = z.scores + align256(decode ? sizeof(double) * 2 * (size_t)n_experts : 0);
+    z.bytes = z.gu_part + (decode ? gu_part_bytes(std::min(n_tokens, kDecSplitMaxTokens), dec_inter) : 0);
+    return z;
 }
 
 // ---------------------------------------------------------------------------

@@ -14,9 +14,9 @@ SOURCE = r"""
 #include "cx_shapes.h"
 using namespace cx;
 extern "C" {
-void expert(int t, int h, int i, int lds, size_t* out) {
-    const ExpertScratch z = expert_scratch(t, h, i, lds);
-    out[0] = z.h_hi; out[1] = z.h_lo; out[2] = z.gu_part;
+size_t expert(int t, int h, int i, int lds) { return expert_scratch_bytes(t, h, i, lds); }
+size_t call(int t, int h, int i, int lds, int dma) {
+    return expert_call_bytes(expert_route(t, h, i, lds, dma, dma, dma).path, t, i);
 }
 int small(int h, int i) { return expert_small_shape(h, i); }
 size_t few_bytes(int t, int i) { return few_scratch_bytes(t, i); }
@@ -29,7 +29,10 @@ void route(int t, int h, int i, int lds, int x, int gu, int dn, int* out) {
 int big(int h, int i, int n, int sh) { return big_min_pairs(h, i, n, sh, 256); }
 int few_lds(int t) { return few_gu_lds(few_tiles(t)); }
 int slices(int t, int h, int e) { return route_slices(t, h, e); }
-size_t part(int t, int h, int e) { return route_part_cells(t, h, e); }
+void router(int t, int h, int e, int decode, int inter, size_t* out) {
+    const RouteScratch z = route_scratch(t, h, e, decode, inter);
+    out[0] = z.part; out[1] = z.scores; out[2] = z.gu_part; out[3] = z.bytes;
+}
 size_t buffer(int t, int k, int e, int sh) { return plan_buffer_bytes(t, k, e, sh); }
 size_t plan(int t, int k, int e, int sh, int cap, int dense) {
     PlanSizes z = plan_sizes(t, k, e, sh);
@@ -47,7 +50,7 @@ def rules(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{CSRC}",
                     str(d / "rules.cc"), "-o", str(d / "rules.so")], check=True)
     L = C.CDLL(str(d / "rules.so"))
-    for f in ("few_bytes", "part", "buffer", "plan"):
+    for f in ("few_bytes", "expert", "call", "buffer", "plan"):
         getattr(L, f).restype = C.c_size_t
     return L
 
@@ -55,18 +58,20 @@ def rules(tmp_path_factory):
 @pytest.mark.parametrize("lds", [160 << 10, 64 << 10])
 @pytest.mark.parametrize("H,I", [(7168, 2048), (1024, 512), (512, 512), (7168, 512), (4096, 1536), (2048, 768)])
 def test_expert_scratch_never_shrinks(rules, H, I, lds):
-    last = (0, 0, 0)
+    last = 0
     for T in range(1, 700):
-        out = (C.c_size_t * 3)()
-        rules.expert(T, H, I, lds, out)
-        got = tuple(out)
-        assert all(a <= b for a, b in zip(last, got)), (T, last, got)
+        got = rules.expert(T, H, I, lds)
+        assert got >= last, (T, last, got)
         last = got
-        if T <= 4 and rules.small(H, I):
-            need = (0, 0, 16 * T * I)  # two k-parts of gate and up, fp32
-        else:
-            need = (max(2 * T * I, rules.few_bytes(T, I) if rules.few(H, I, T, lds) else 0), 2 * T * I, 0)
-        assert all(n <= b for n, b in zip(need, got)), (T, need, got)
+        for dma in (0, 1):
+            need = rules.call(T, H, I, lds, dma)
+            if T <= 4 and rules.small(H, I):
+                assert need == 16 * T * I  # two k-parts of gate and up, fp32
+            elif dma and rules.few(H, I, T, lds):
+                assert need == rules.few_bytes(T, I)
+            else:
+                assert need == (2 * T * I + 255) // 256 * 256 + 2 * T * I
+            assert need <= got, (T, need, got)
 
 
 @pytest.mark.parametrize("lds", [160 << 10, 96 << 10, 64 << 10, 16 << 10])
@@ -102,12 +107,20 @@ def test_wide_loads_only_from_aligned_rows(rules, H, I):
 
 
 @pytest.mark.parametrize("H,E", [(7168, 256), (1024, 64), (640, 72), (384, 40), (1000, 8)])
-def test_router_slices_never_shrink(rules, H, E):
+@pytest.mark.parametrize("decode,inter", [(0, 0), (1, 0), (1, 512)])
+def test_router_scratch_never_shrinks(rules, H, E, decode, inter):
     last = 0
     for T in range(1, 600):
-        got = rules.part(T, H, E)
-        assert got >= last and got >= rules.slices(T, H, E) * T * E, T
-        last = got
+        out = (C.c_size_t * 4)()
+        rules.router(T, H, E, decode, inter, out)
+        part, scores, gu, end = out
+        assert end >= last, T
+        last = end
+        assert not any(p % 256 for p in (part, scores, gu)) and part >= 8 * T * E
+        if T > 16 or not decode:
+            assert scores - part >= 8 * rules.slices(T, H, E) * T * E, T
+        if decode:
+            assert gu - scores >= 16 * E and end - gu >= 16 * min(T, 8) * inter, T
 
 
 @pytest.mark.parametrize("H,I,n,shared,pairs", [
