@@ -279,7 +279,6 @@ __device__ __forceinline__ void gate_up_tile_body(const ExpertLaunch& L, int til
         }
         if (q < u.np && 4 * g < TR) {
             const size_t p = (size_t)(u.pb + q);
-            const float wf = !SINGLE && L.fold_weight ? L.plan.pair_weight[p] : 1.0f;
             const int row = r0 + 4 * g;
             uint32_t hi[4], lo[4];
             float hv[4];
@@ -288,9 +287,8 @@ __device__ __forceinline__ void gate_up_tile_body(const ExpertLaunch& L, int til
                 const float gate = G[i], up = U[i];
                 const float h = (gate / (1.0f + expf(-gate))) * up;
                 hv[i] = h;
-                const float hw = h * wf;
-                hi[i] = bf16_rne(hw);
-                lo[i] = bf16_rne(hw - __uint_as_float(hi[i] << 16));
+                hi[i] = bf16_rne(hv[i]);
+                lo[i] = bf16_rne(hv[i] - __uint_as_float(hi[i] << 16));
             }
             *reinterpret_cast<uint2*>(L.h_hi + p * I + row) =
                 uint2{hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16)};

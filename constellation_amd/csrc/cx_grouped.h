@@ -238,14 +238,12 @@ __device__ __forceinline__ void grp_gate_up_item(const ExpertLaunch& L, const Un
     };
     grp_stream<NKB, D, PS>(issue, publish, compute,
                            [&] { asm volatile("" : "+v"(scg_v), "+v"(scu_v)); });
-    // epilogue: h = SiLU(gate) * up as bf16 hi + lo (route weight folded in
-    // when the caller combines by plain sums)
+    // epilogue: h = SiLU(gate) * up as bf16 hi + lo
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
         const int q = tt * kTileTok + c;
         if (q < u.np) {
             const size_t p = (size_t)(u.pb + q);
-            const float wf = !SINGLE && L.fold_weight ? L.plan.pair_weight[p] : 1.0f;
             const int row = r0 + 4 * g;
             uint32_t hi[4], lo[4];
             float hv[4];
@@ -254,9 +252,8 @@ __device__ __forceinline__ void grp_gate_up_item(const ExpertLaunch& L, const Un
                 const float gate = accg[tt][i], up = accu[tt][i];
                 const float h = (gate / (1.0f + expf(-gate))) * up;
                 hv[i] = h;
-                const float hw = h * wf;
-                hi[i] = bf16_rne(hw);
-                lo[i] = bf16_rne(hw - __uint_as_float(hi[i] << 16));
+                hi[i] = bf16_rne(hv[i]);
+                lo[i] = bf16_rne(hv[i] - __uint_as_float(hi[i] << 16));
             }
             *reinterpret_cast<uint2*>(L.h_hi + p * I + row) = uint2{hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16)};
             *reinterpret_cast<uint2*>(L.h_lo + p * I + row) = uint2{lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16)};
@@ -398,7 +395,6 @@ __device__ __forceinline__ void grp_gate_up_item_c1(const ExpertLaunch& L, const
     }
     if (c < u.np) {
         const size_t p = (size_t)(u.pb + c);
-        const float wf = !SINGLE && L.fold_weight ? L.plan.pair_weight[p] : 1.0f;
         const int row = r0 + 4 * g;
         uint32_t hi[4], lo[4];
         float hv[4];
@@ -407,9 +403,8 @@ __device__ __forceinline__ void grp_gate_up_item_c1(const ExpertLaunch& L, const
             const float gate = accg[i], up = accu[i];
             const float h = (gate / (1.0f + expf(-gate))) * up;
             hv[i] = h;
-            const float hw = h * wf;
-            hi[i] = bf16_rne(hw);
-            lo[i] = bf16_rne(hw - __uint_as_float(hi[i] << 16));
+            hi[i] = bf16_rne(hv[i]);
+            lo[i] = bf16_rne(hv[i] - __uint_as_float(hi[i] << 16));
         }
         *reinterpret_cast<uint2*>(L.h_hi + p * I + row) = uint2{hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16)};
         *reinterpret_cast<uint2*>(L.h_lo + p * I + row) = uint2{lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16)};

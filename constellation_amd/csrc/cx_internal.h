@@ -168,7 +168,6 @@ struct ExpertLaunch {
     void* y;                      // single mode: [T, hidden] out dtype
     float* y_f32;                 // single mode / fused decode: optional fp32 output
     int out_dtype;
-    int fold_weight;              // phase A multiplies h by the pair's route weight
     int np_lds;                   // >0: stage up to np_lds activation rows (x dma_aligned) per item in LDS
     int skip_shared;              // grouped mode: routed items only (shared expert done apart)
     int max_lds;                  // dynamic LDS per workgroup the device allows (0: unknown)

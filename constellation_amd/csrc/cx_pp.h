@@ -434,7 +434,6 @@ __device__ __forceinline__ void pp_gate_up_item(const ExpertLaunch& L, const Uni
     for (int tt = 0; tt < NT; ++tt) {
         const int q = tt * kTileTok + c;
         if (q >= u.np) continue;
-        const float wf = !SINGLE && L.fold_weight ? L.plan.pair_weight[u.pb + q] : 1.0f;
         const size_t o = (size_t)(u.pb + q) * I + r0 + 4 * g;
         uint32_t hi[4], lo[4];
         float hv[4];
@@ -443,9 +442,8 @@ __device__ __forceinline__ void pp_gate_up_item(const ExpertLaunch& L, const Uni
             const float gate = acc[0][tt][i], up = acc[1][tt][i];
             const float hh = (gate / (1.0f + expf(-gate))) * up;
             hv[i] = hh;
-            const float hw = hh * wf;
-            hi[i] = bf16_rne(hw);
-            lo[i] = bf16_rne(hw - __uint_as_float(hi[i] << 16));
+            hi[i] = bf16_rne(hv[i]);
+            lo[i] = bf16_rne(hv[i] - __uint_as_float(hi[i] << 16));
         }
         *reinterpret_cast<uint2*>(L.h_hi + o) = uint2{hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16)};
         *reinterpret_cast<uint2*>(L.h_lo + o) = uint2{lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16)};
