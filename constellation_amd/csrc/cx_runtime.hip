@@ -232,7 +232,7 @@ struct cx_ctx {
     int max_lds = 65536;               // dynamic LDS budget per workgroup
     int n_cu = 0;                      // compute units (0: unknown)
     DevBuf plan_buf, hhi, hlo, ypart, route_ids, route_w;
-    DevBuf one;                        // scratch of one expert (expert_scratch_bytes)
+    DevBuf one, one_lo;                // scratch of one expert (ExpertScratch)
     DevBuf logits;                     // router scratch (RouteScratch), the logits first
     int route_T = 0, route_E = 0;      // shape of the fp64 logits of the last router call
     DevBuf dx, dy;                     // cx_expert_run_host staging (device)
@@ -400,9 +400,9 @@ ExpertPlan plan_expert(const cx_expert_desc& e, const void* x, int in_dtype, int
 }
 
 // Launches a planned expert on `s` with P.scratch_bytes of scratch (256-byte
-// aligned).  ctx (nullable) only collects timing.
+// aligned); h_lo: the lo plane of the tile paths.  ctx (nullable) only collects timing.
 int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* x, int in_dtype,
-               int n_tokens, void* y, int out_dtype, float* y_f32, void* scratch, hipStream_t s) {
+               int n_tokens, void* y, int out_dtype, float* y_f32, void* scratch, void* h_lo, hipStream_t s) {
     if (P.route.path == kPathGeneric) {
         CX_HIP(launch_generic_expert(e, x, in_dtype, n_tokens, static_cast<float*>(scratch), y, out_dtype, y_f32, s));
         return CX_OK;
@@ -419,7 +419,7 @@ int run_expert(cx_ctx* ctx, ExpertPlan& P, const cx_expert_desc& e, const void* 
         return CX_OK;
     }
     L.h_hi = static_cast<uint16_t*>(scratch);
-    L.h_lo = reinterpret_cast<uint16_t*>(static_cast<char*>(scratch) + h_lo_offset(n_tokens, e.inter));  // (not few)
+    L.h_lo = static_cast<uint16_t*>(h_lo);
     if (P.route.path == kPathFew) {
         {
             Span sp(ctx, "gate_up", s);
@@ -1054,7 +1054,7 @@ int cx_ctx_destroy(cx_ctx* c) {
     (void)hipSetDevice(c->device);
     (void)hipDeviceSynchronize();
     drain_spans(c);
-    DevBuf* bufs[] = {&c->plan_buf, &c->hhi, &c->hlo, &c->ypart, &c->one, &c->logits, &c->route_ids,
+    DevBuf* bufs[] = {&c->plan_buf, &c->hhi, &c->hlo, &c->ypart, &c->one, &c->one_lo, &c->logits, &c->route_ids,
                       &c->route_w, &c->dx, &c->dy};
     for (DevBuf* b : bufs)
         if (b->p) (void)hipFree(b->p);
@@ -1118,11 +1118,12 @@ int cx_expert_run(cx_ctx* ctx, const cx_expert_desc* expert, const void* x, int 
     if ((rc = set_device(ctx->device))) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     ExpertPlan P = plan_expert(*expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->max_lds, ctx->n_cu);
-    const size_t bytes = P.route.path == kPathGeneric
-                             ? P.scratch_bytes
-                             : expert_scratch_bytes(n_tokens, expert->hidden, expert->inter, ctx->max_lds);
-    if ((rc = ensure(&ctx->one, bytes, s))) return rc;
-    return run_expert(ctx, P, *expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->one.p, s);
+    const ExpertScratch z = P.route.path == kPathGeneric
+                                ? ExpertScratch{P.scratch_bytes, 0}
+                                : expert_scratch(n_tokens, expert->hidden, expert->inter, ctx->max_lds);
+    if ((rc = ensure(&ctx->one, z.bytes, s)) || (z.lo_bytes && (rc = ensure(&ctx->one_lo, z.lo_bytes, s)))) return rc;
+    return run_expert(ctx, P, *expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, ctx->one.p,
+                      z.lo_bytes ? ctx->one_lo.p : static_cast<char*>(ctx->one.p) + h_lo_offset(n_tokens, expert->inter), s);
 }
 
 int cx_expert_run_static(int device, const cx_expert_desc* expert, const void* x, int in_dtype,
@@ -1144,7 +1145,7 @@ int cx_expert_run_static(int device, const cx_expert_desc* expert, const void* x
                     "more than the static %d (use cx_expert_run)",
                     n_tokens, expert->inter, need, (int)CX_STATIC_SCRATCH_BYTES);
     return run_expert(nullptr, P, *expert, x, in_dtype, n_tokens, y, out_dtype, y_f32, base,
-                      static_cast<hipStream_t>(stream));
+                      base + h_lo_offset(n_tokens, expert->inter), static_cast<hipStream_t>(stream));
 }
 
 int cx_expert_run_host(cx_ctx* ctx, const cx_expert_desc* expert, const void* x_host,

@@ -158,12 +158,20 @@ inline size_t expert_call_bytes(ExpertPath path, int n_tokens, int inter) {
 }
 
 // The same of a context, for the paths of all calls with up to n_tokens tokens.
-inline size_t expert_scratch_bytes(int n_tokens, int hidden, int inter, int max_lds) {
+// Above kFewMaxTokens tokens the lo plane has a buffer of its own (a first call of
+// 300 tokens took 78 us with two allocations of 1.2 MB and 89 to 114 with one of 2.4).
+struct ExpertScratch {
+    size_t bytes, lo_bytes;
+};
+
+inline ExpertScratch expert_scratch(int n_tokens, int hidden, int inter, int max_lds) {
     const bool small = expert_small_shape(hidden, inter);
-    const int few = std::min(n_tokens, few_max_tokens(max_lds));
-    return std::max({small ? expert_call_bytes(kPathSmall, std::min(n_tokens, kDownKsRows), inter) : 0,
-                     few_ok(hidden, inter, few, max_lds) ? expert_call_bytes(kPathFew, few, inter) : 0,
-                     small && n_tokens <= kDownKsRows ? 0 : expert_call_bytes(kPathTiles, n_tokens, inter)});
+    const int few = std::min(n_tokens, few_max_tokens(max_lds)), both = std::min(n_tokens, kFewMaxTokens);
+    const size_t plane = n_tokens > both ? (size_t)n_tokens * inter * 2 : 0;
+    return {std::max({small ? expert_call_bytes(kPathSmall, std::min(n_tokens, kDownKsRows), inter) : 0,
+                      few_ok(hidden, inter, few, max_lds) ? expert_call_bytes(kPathFew, few, inter) : 0,
+                      small && n_tokens <= kDownKsRows ? 0 : expert_call_bytes(kPathTiles, both, inter), plane}),
+            plane};
 }
 
 // ---------------------------------------------------------------------------
