@@ -1,7 +1,8 @@
-// cx_pp.h — the grouped fp8 expert MLP as two LDS-ring GEMM kernels whose two
-// waves per SIMD alternate between loading and multiplying (ping-pong), for
-// items of up to 128 pairs: prefill chunks with many tokens per expert, and one
-// expert over more than 16 tokens.
+// cx_pp.h — the grouped fp8 expert MLP as two GEMM kernels on a ring of LDS stages
+// whose two waves per SIMD alternate between loading and multiplying (ping-pong),
+// for items of up to 128 pairs: prefill chunks with many tokens per expert
+// (big_min_pairs), and one expert over more than 64 tokens (more than 16 at widths
+// without few-token kernels).
 // Semantics: RunFusedUpGateReferenceV2 / RunDownReferenceV2
 // (expert_node_v2/backend/expert_reference_v2.cc:11-144) per expert,
 // dequantise-then-fp32, h kept to 16 significant bits (bf16 hi + lo).

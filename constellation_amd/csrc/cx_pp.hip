@@ -21,8 +21,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
 // the least rounds x time, the larger of equals (fewer reads of the weights).
 // us[n - 1]: an item of n column tiles alone on its CU at hidden 7168, inter
 // 2048, from 17 to 4096 tokens of one expert at every count; only their ratios
-// matter.  At 300 tokens gate/up takes 35 us with 2 tiles and 43 with 4, down
-// 23 with 3 and 35 with 2; at 1500 80 with 6 and 96 with 4.
+// matter (rows of other lengths take the same counts; at ten shapes from 512 x 512
+// to 4096 x 1536 no call of 17 to 4096 tokens was slower than with the 64-token items
+// before).  At 300 tokens gate/up takes 35 us with 2 tiles and 43 with 4, down 23
+// with 3 and 35 with 2; at 1500 80 with 6 and 96 with 4.
 constexpr int kPpUsGu[kPpMaxTiles] = {27, 33, 40, 43, 56, 65, 74, 84};
 constexpr int kPpUsDn[kPpMaxTiles] = {13, 17, 22, 24, 38, 38, 45, 45};
 

@@ -8,10 +8,11 @@
 // the exact-math decision; ties break toward the lower index.
 //
 // Launch shapes
-//  * cx_route / general path: k_route_logits_split (4 to 256 tokens) or
-//    k_route_logits_mfma (more), on the fp64 matrix cores, or k_route_logits (one
-//    workgroup per expert row streams W_r once for up to 16 tokens; fewer, or
-//    other widths), then k_route_select (4 tokens per workgroup), then, for the grouped MoE, k_plan (up to 64 workgroups).
+//  * cx_route / general path: k_route_logits_split (from 4 tokens, up to 256
+//    tiles) or k_route_logits_mfma (more), on the fp64 matrix cores, or
+//    k_route_logits (one workgroup per expert row streams W_r once for up to 16
+//    tokens; fewer tokens, or other widths), then k_route_select (4 tokens per
+//    workgroup), then, for the grouped MoE, k_plan (up to 64 workgroups).
 //  * decode pipeline (T <= 16, E <= 256):
 //      stage 1  k_dec_logits        router logits
 //      stage 2  k_dec_select_sgu    selection + planner (workgroup 0) |
@@ -1240,10 +1241,10 @@ __global__ __launch_bounds__(64 * kLgWaves) void k_route_logits_mfma(FusedArgs A
     }
 }
 
-// Router logits for 4 to 256 tokens: tiles of 16 experts x 16 tokens with K
+// Router logits for few to medium calls (route_slices): tiles of 16 experts x 16 tokens with K
 // split over S grid slices and the 4 waves of each (one accumulator for the even
-// and one for the odd MFMA steps), so that up to 256 workgroups share the
-// products: the 16 x 32 tiles above left 224 of 256 CUs idle at 64 tokens and
+// and one for the odd MFMA steps), so that 256 workgroups share the products at 256
+// experts (the slices follow from the tokens alone; fewer experts have fewer): the 16 x 32 tiles above left 224 of 256 CUs idle at 64 tokens and
 // spent 24 us of matrix time on the others, and a workgroup per expert row reads
 // every token's x once per expert.  Slice z writes its sums to part[z][t][e]; the
 // selection adds them up in the order of z.  256 experts, hidden 7168, us a router

@@ -243,12 +243,13 @@ def test_small_batch_expert_full_size(gpu, oracle, in_dt):
         e.free()
 
 
-@pytest.mark.parametrize("T,dt", [(17, FP16), (129, BF16), (300, FP16), (700, BF16), (1100, BF16), (2000, FP16)])
+@pytest.mark.parametrize("T,dt", [(17, FP16), (65, BF16), (129, BF16), (300, FP16), (700, BF16), (1100, BF16), (2000, FP16)])
 def test_many_tokens_one_expert_full_size(gpu, oracle, T, dt):
-    """More than 16 tokens take the ping-pong GEMM, whose items have 1 (17 tokens)
-    to 8 (2000) column tiles by the token count; the last item is partial.  Each
-    token against the oracle-tested 16-token path, the first, last and a middle
-    one against the oracle."""
+    """More than 64 tokens take the ping-pong GEMM, whose items have 1 (gate/up of 65
+    and 129 tokens) to 8 (2000) column tiles by the token count; the last item is
+    partial (17 tokens take the few-token kernels).  Each token against the
+    oracle-tested 16-token path, the first, last and a middle one against the
+    oracle."""
     print(f"[expert] many tokens T={T}", flush=True)
     from constellation_amd.engine import Expert
     e = Expert.generate(0, 91, 0x740)

@@ -2,8 +2,8 @@
 cx_gen_expert writes) against the same bytes row-major: the resident bytes
 read back equal, and every kernel path that reads gate/up gives bit-identical
 outputs (one expert at 1..40 tokens; layers mixing both layouts through the
-one-token pipeline, the decode pipeline, the grouped prefill GEMM and the
-LDS-ring GEMM)."""
+one-token pipeline, the decode pipeline, the 64-pair grouped GEMM and the
+ping-pong GEMM)."""
 import numpy as np
 import pytest
 import torch
@@ -130,8 +130,8 @@ def test_generated_expert_is_tiled_and_matches_row_major_upload(gpu):
 @pytest.mark.parametrize("T,K,E", [(1, 8, 32), (5, 8, 32), (16, 8, 32), (70, 8, 32), (200, 4, 4)])
 def test_layer_mixing_layouts_equals_row_major_layer(gpu, T, K, E):
     """Routes given (cx_moe): T = 1 the one-token down + combine, T <= 16 the
-    decode pipeline, 70 the grouped GEMM, 200 x 4 routes over 4 experts the
-    LDS-ring GEMM (>= 128 pairs per expert).  Experts alternate tiled and
+    decode pipeline, 70 the 64-pair grouped GEMM, 200 x 4 routes over 4 experts the
+    ping-pong GEMM (200 pairs per expert).  Experts alternate tiled and
     row-major; the reference layer holds the same bytes all row-major."""
     print(f"[layout] layer T={T} K={K} E={E}", flush=True)
     from constellation_amd.engine import Layer

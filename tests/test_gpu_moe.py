@@ -191,7 +191,7 @@ def test_moe_grouped_vs_oracle(gpu, oracle, T, prefill, I):
     (1024, 2048, 6, 200, 4, torch.bfloat16, True)])
 def test_moe_many_tokens_per_expert(gpu, oracle, H, I, E, T, K, dtype, shared):
     """Calls with >= 128 pairs per routed expert on average take 128-pair
-    items through the LDS-ring GEMM: experts cut into a full item plus a
+    items through the ping-pong GEMM, at any shape: experts cut into a full item plus a
     partial one, or a single partial item; hidden of 8 and 16 k-blocks,
     inter of 4, 8 and 16; bf16 and fp16 activations.  Every token against
     the oracle."""
@@ -356,7 +356,7 @@ def test_layer_rows_that_start_between_16_bytes(gpu, H, I, E, Ts):
 
 def test_many_tokens_per_resident_expert(gpu, oracle):
     """A node's share: 4 of 16 experts resident, 160 tokens x 4 routes over
-    them (160 pairs per resident expert), so the LDS-ring GEMM serves the call
+    them (160 pairs per resident expert), so the ping-pong GEMM serves the call
     although 640 routes are few for all 16 slots.  Every token against the
     oracle; the layer table's empty slots are never read."""
     print("[moe] many tokens per resident expert", flush=True)
@@ -388,9 +388,8 @@ def test_many_tokens_per_resident_expert(gpu, oracle):
 
 
 def test_planner_many_routes_vs_oracle(gpu, oracle):
-    """4800 routes (1200 tokens x 4): more than the planner held in LDS as
-    32-bit ids; staged as 16-bit ids with the validity bits in registers.
-    Every token against the oracle (shared expert on, the LDS-ring GEMM)."""
+    """4800 routes (1200 tokens x 4): a plan of five workgroups.  Every token
+    against the oracle (shared expert on, the ping-pong GEMM)."""
     print("[moe] planner 4800 routes", flush=True)
     E, H, I, T, K = 8, 1024, 512, 1200, 4
     layer, experts, sh, cpu, cpu_sh = _make_layer(gpu, oracle, E, H, I, seed=64, shared=True)
@@ -412,10 +411,10 @@ def test_planner_many_routes_vs_oracle(gpu, oracle):
 
 
 def test_planner_beyond_staging_matches_chunks(gpu, oracle):
-    """68,000 routes (17,000 tokens x 4) exceed what the staged planner holds
-    (64 per thread) and take the general planner; the same routes in four
-    chunks take the staged one.  A pair's value does not depend on its item's
-    other pairs, so the outputs are bit-identical."""
+    """68,000 routes (17,000 tokens x 4): 64 planner workgroups, the most there
+    are, with more than 1024 routes each; the same routes in four chunks of 17
+    workgroups.  A pair's value does not depend on its item's other pairs, so the
+    outputs are bit-identical."""
     print("[moe] planner beyond staging", flush=True)
     E, H, I, T, K = 4, 1024, 512, 17000, 4
     layer, experts, sh, cpu, cpu_sh = _make_layer(gpu, oracle, E, H, I, seed=67, shared=False)
@@ -439,7 +438,7 @@ def test_planner_beyond_staging_matches_chunks(gpu, oracle):
 
 
 def test_full_size_many_tokens_per_expert(gpu, oracle):
-    """DeepSeek-V3 shapes (H=7168, I=2048) through the LDS-ring GEMM: 8
+    """DeepSeek-V3 shapes (H=7168, I=2048) through the ping-pong GEMM: 8
     routed experts + shared, 256 tokens x 4 routes (128 pairs per expert on
     average).  Every token against the oracle fed the device-resident
     weights, and against the decode pipeline."""

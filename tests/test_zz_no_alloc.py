@@ -41,7 +41,7 @@ def _run_ctx(gpu, e, x, out_dt):
 
 @pytest.mark.parametrize("in_dt,out_dt", [(BF16, BF16), (FP16, FP16)])
 def test_static_matches_context_path_full_size(gpu, in_dt, out_dt):
-    """DeepSeek-V3 expert (7168 x 2048): the tile path (8 tokens) and then the
+    """DeepSeek-V3 expert (7168 x 2048): the few-token path (8 tokens) and then the
     small k-part path (3 tokens), back to back on the shared array."""
     from constellation_amd._lib import CX_OK
     from constellation_amd.engine import Expert
@@ -144,7 +144,7 @@ def test_static_under_graph_capture(gpu, T):
     launches only: the first, eager call has looked up the static array),
     replayed three times on new inputs with eager work and syncs between the
     replays; every replay equals cx_expert_run bit for bit.  T = 1 takes the
-    k-part path, T = 8 the tile path."""
+    k-part path, T = 8 the few-token path."""
     from constellation_amd._lib import CX_OK
     from constellation_amd.engine import Expert
     print(f"[no_alloc] graph capture T={T}", flush=True)
