@@ -103,17 +103,19 @@ inline bool grp_shape(int hidden, int inter) {
 //   64, none shared  535 598 708 904 1132 1514   523 569 622 741 816 1276
 // The shared expert's items, all full, run last: where the others last for few
 // rounds of the CUs, 128 pairs at the end cost more than fewer reads of the weights
-// save, up to 79 pairs (8 experts, which fit one round, gain from 20: 121 / 105).
-// Rows of few blocks gain as late, a ring's fill and drain being a larger part of an
-// item: 512 x 7168 (inter x hidden), 256 experts 683 765 908 1171 1488 and 732 807
-// 936 1048 1181; and below two rounds the halved count of workgroups shows too (1024
-// x 512, 16 experts, 96 pairs 45 against 52), up to the 128 pairs of a full item.
+// save, up to 63 pairs (8 experts, which fit one round, gain from 20: 121 / 105; 4
+// gain up to 48, 121 / 117, and from 80, but lose between, 125 / 142 at 64).
+// Rows of few blocks gain later, a ring's fill and drain being a larger part of an
+// item, and the later the fewer the experts, as the halved count of items leaves CUs
+// idle: 7168 x 512 (hidden x inter), 256 experts 683 765 908 1171 1488 2070 and 732
+// 807 936 1048 1181 1728; 64 / 80 / 96 pairs of 1024 x 512, 64 experts 76 91 109 and
+// 86 91 96, 16 experts 44 45 44 and 51 47 51.
 constexpr int kBigPairs = 128;
 inline int big_min_pairs(int hidden, int inter, int n_resident, bool shared, int n_cu) {
     if (!grp_shape(hidden, inter)) return 20;
     const int wgs = (n_resident + (shared ? 1 : 0)) * (inter / kPpRowsGu);  // gate/up, an item each
-    if (hidden / kKB == 56 && inter / kKB == 16) return !shared || wgs <= n_cu || wgs >= 8 * n_cu ? 20 : 80;
-    return wgs >= 2 * n_cu ? 80 : kBigPairs;
+    if (hidden / kKB == 56 && inter / kKB == 16) return !shared || wgs <= n_cu || wgs >= 8 * n_cu ? 20 : 64;
+    return n_resident >= 256 ? 64 : n_resident >= 32 ? 80 : kBigPairs;
 }
 
 // Kernels of one expert on the fast paths.  Above 16 tokens the 64-token items of

@@ -98,7 +98,7 @@ def _smaller_calls(gpu, kind, H, I, E):
     def call(T, c):
         y, _, ids, w = c.moe_layer(layer, x[:T], w_r, bias, **opt)
         return y, ids, w
-    return 1100, (1024, 1023, 300, 40, 17, 16, 8, 1), call, free  # 128-pair items from 1024
+    return 1100, (640, 639, 300, 40, 17, 16, 8, 1), call, free  # 128-pair items from 640
 
 
 @pytest.mark.parametrize("kind", ["route", "expert", "layer"])

@@ -132,8 +132,8 @@ def test_router_scratch_never_shrinks(rules, H, E, decode, inter):
 
 @pytest.mark.parametrize("H,I,n,shared,pairs", [
     (7168, 2048, 256, 1, 20), (7168, 2048, 127, 1, 20), (7168, 2048, 64, 0, 20), (7168, 2048, 4, 0, 20),
-    (7168, 2048, 64, 1, 80), (7168, 2048, 16, 1, 80), (7168, 2048, 15, 1, 20),  # the shared expert's items last
-    (7168, 512, 256, 1, 80), (1024, 2048, 64, 0, 80), (1024, 512, 64, 1, 128), (512, 512, 8, 0, 128),  # few blocks
+    (7168, 2048, 64, 1, 64), (7168, 2048, 16, 1, 64), (7168, 2048, 15, 1, 20),  # the shared expert's items last
+    (7168, 512, 256, 1, 64), (7168, 512, 255, 1, 80), (1024, 2048, 64, 0, 80), (1024, 512, 32, 1, 80), (512, 512, 31, 0, 128),  # few blocks
     (2048, 768, 128, 1, 20), (4096, 1536, 8, 1, 20), (2048, 512, 64, 1, 20)])  # no 64-pair kernels
 def test_pairs_per_expert_of_128_pair_items(rules, H, I, n, shared, pairs):
     """The least pairs per resident expert for 128-pair items, on 256 CUs."""
